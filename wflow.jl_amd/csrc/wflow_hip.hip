@@ -193,6 +193,20 @@ struct RouteArgs {
     double dts_s[2], dts_l[2], dts_r[2];  // sub-step lengths: first (S-1) steps and the last one
 };
 
+// A kernel's arguments read where they are used. Passed by value, Dev is some 200 pointers that the
+// compiler loads once at the start of a persistent kernel; they do not fit the scalar registers,
+// so they are parked in lanes of vector registers and every use takes them out again, a
+// v_readlane (about 5 cycles) per half pointer: 2261 of them in k_route<4>. The argument pointer is
+// laundered here once per chunk instead, so the loads (one scalar load for up to eight pointers,
+// from the constant cache) stay behind it, in the chunk. `Args` mirrors the kernel's parameter list
+// (explicit arguments start at offset 0 of the argument segment, each at its own alignment).
+template <class Args>
+__device__ __forceinline__ const Args& kernel_args() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const Args*)p;
+}
+
 // State of the adaptive sub-steps (one launch per sub-step and family), kept between launches.
 struct AdArgs {
     double* szi;           // [n] subsurface water table depth
@@ -209,6 +223,18 @@ struct AdArgs {
                                          // order of the reference's river topological sort
     const int* chain_r;    // [nchunks_r] 1: a chain chunk (see run_chain)
     int nchunks_r;
+};
+
+struct RouteKernelArgs {
+    Dev d;
+    RouteArgs a;
+};
+struct AdKernelArgs {
+    Dev d;
+    RouteArgs a;
+    AdArgs x;
+    double dts;
+    int first, last;
 };
 
 // Order-statistic selection over 64-bit keys (the bit patterns of positive doubles order as
@@ -1116,8 +1142,8 @@ __device__ __forceinline__ void total_storage_finish(const Dev& d, const int p, 
 // well, from the step's forcing frame, and the arrays the steps hand on are accessed coherently.
 // A chunk's step can thus run while the long chains of the previous step are still draining.
 template <int N, bool EXT, bool MULTI = false, bool FUSE = false>
-__global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_eu(route_waves(N)))) k_route(Dev d,
-                                                                                                    RouteArgs a) {
+__global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_eu(route_waves(N)))) k_route(
+    const Dev d_arg, const RouteArgs a_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
     __shared__ int x_k[ROUTE_BLOCK];     // per-wave exchange tables of the routing families
     __shared__ double x_q[ROUTE_BLOCK];
@@ -1125,11 +1151,15 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
     const int wbase = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~(WAVE - 1)));
     int* const lds_k = x_k + wbase;
     double* const lds_q = x_q + wbase;
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[a.parity ^ 1] = 0ull;  // next launch's counter
-    const int n = d.n;
-    const double dt = d.dt;
-    const unsigned long long tickets = (unsigned long long)a.nchunks * (MULTI ? (unsigned long long)a.nsteps : 1ull);
+    if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;  // next launch's counter
     for (;;) {
+        const RouteKernelArgs& args = kernel_args<RouteKernelArgs>();
+        const Dev& d = args.d;
+        const RouteArgs& a = args.a;
+        const int n = d.n;
+        const double dt = d.dt;
+        const unsigned long long tickets =
+            (unsigned long long)a.nchunks * (MULTI ? (unsigned long long)a.nsteps : 1ull);
         unsigned long long t = 0;
         if (lane == 0) t = atomicAdd(&a.counters[a.parity], 1ull);
         t = __shfl(t, 0);
@@ -1387,16 +1417,23 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
 
 // One subsurface sub-step of length dts (first: the step's first sub-step, last: its last).
 template <int N>
-__global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ssf(Dev d, RouteArgs a, AdArgs x, double dts, int first,
-                                                        int last) {
+__global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ssf(const Dev d_arg, const RouteArgs a_arg,
+                                                        const AdArgs x_arg, const double dts_arg, const int first_arg,
+                                                        const int last_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
     __shared__ int x_k[ROUTE_BLOCK];
     __shared__ double x_q[ROUTE_BLOCK];
     int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
     double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[a.parity ^ 1] = 0ull;
-    const int n = d.n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
+        const AdKernelArgs& args = kernel_args<AdKernelArgs>();
+        const Dev& d = args.d;
+        const RouteArgs& a = args.a;
+        const AdArgs& x = args.x;
+        const double dts = args.dts;
+        const int first = args.first, last = args.last;
+        const int n = d.n;
         AD_TICKET(a.nchunks)
         const int p = c * WAVE + lane;
         const bool valid = p < n;
@@ -1490,16 +1527,23 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ssf(Dev d, RouteArgs a, AdAr
 }
 
 // One overland sub-step of length dts.
-__global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ol(Dev d, RouteArgs a, AdArgs x, double dts, int first,
-                                                       int last) {
+__global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ol(const Dev d_arg, const RouteArgs a_arg,
+                                                        const AdArgs x_arg, const double dts_arg, const int first_arg,
+                                                        const int last_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
     __shared__ int x_k[ROUTE_BLOCK];
     __shared__ double x_q[ROUTE_BLOCK];
     int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
     double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[a.parity ^ 1] = 0ull;
-    const int n = d.n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
+        const AdKernelArgs& args = kernel_args<AdKernelArgs>();
+        const Dev& d = args.d;
+        const RouteArgs& a = args.a;
+        const AdArgs& x = args.x;
+        const double dts = args.dts;
+        const int first = args.first, last = args.last;
+        const int n = d.n;
         AD_TICKET(a.nchunks)
         const int p = c * WAVE + lane;
         const bool valid = p < n;
@@ -1647,16 +1691,23 @@ __device__ __forceinline__ double fp_capacity(const Dev& d, const int r, const i
 // on, in the reference's river topological order, to its floodplain storage, passes on
 // min(storage / dt, capacity) and keeps the rest.
 template <bool RES, bool FP, bool LINK>
-__global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_riv(Dev d, RouteArgs a, AdArgs x, double dts, int first,
-                                                        int last) {
+__global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_riv(const Dev d_arg, const RouteArgs a_arg,
+                                                        const AdArgs x_arg, const double dts_arg, const int first_arg,
+                                                        const int last_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
     __shared__ int x_k[ROUTE_BLOCK];
     __shared__ double x_q[ROUTE_BLOCK];
     int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
     double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[a.parity ^ 1] = 0ull;
-    const int nr = d.nriv;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
+        const AdKernelArgs& args = kernel_args<AdKernelArgs>();
+        const Dev& d = args.d;
+        const RouteArgs& a = args.a;
+        const AdArgs& x = args.x;
+        const double dts = args.dts;
+        const int first = args.first, last = args.last;
+        const int nr = d.nriv;
         AD_TICKET(x.nchunks_r)
         const int rp = c * WAVE + lane;
         const bool valid = rp < nr;
@@ -1812,16 +1863,19 @@ __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long v)
 // upstream cells pass on, in the reference's topological order, to its own material, passes on
 // min(material / dt, capacity) and keeps the rest. The capacities come from the state before
 // the transport (TAN80 = 5.67, snow_storage_max = 10 m).
-__global__ void __launch_bounds__(ROUTE_BLOCK) k_snow_transport(Dev d, RouteArgs a) {
+__global__ void __launch_bounds__(ROUTE_BLOCK) k_snow_transport(const Dev d_arg, const RouteArgs a_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
     __shared__ int x_k[ROUTE_BLOCK];
     __shared__ double x_q[ROUTE_BLOCK];
     int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
     double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[a.parity ^ 1] = 0ull;
-    const int n = d.n;
-    const double dt = d.dt;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
+        const RouteKernelArgs& args = kernel_args<RouteKernelArgs>();
+        const Dev& d = args.d;
+        const RouteArgs& a = args.a;
+        const int n = d.n;
+        const double dt = d.dt;
         AD_TICKET(a.nchunks)
         const int p = c * WAVE + lane;
         const bool valid = p < n;
