@@ -10,6 +10,15 @@
 #include "wfh_math.h"
 
 #define WFH_HD __host__ __device__ inline
+// for functions that take a column by reference: not inlined, the call would put it into memory
+#define WFH_HD_INLINE __host__ __device__ __attribute__((always_inline)) inline
+
+// True when the condition holds in any lane of the wave that is executing (one cell on the host).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define WFH_ANY(x) __any(x)
+#else
+#define WFH_ANY(x) (x)
+#endif
 
 namespace wfh {
 
@@ -226,46 +235,74 @@ WFH_HD double rwu_reduction_feddes(double h, double h1, double h2, double h3, do
 // ---- kinematic wave ------------------------------------------------------------------------
 // kinematic_wave  Wflow/src/routing/surface/surface_process.jl:24-70
 //
-// Split in two so that a routing loop can hoist everything that does not depend on the
-// upstream inflow q_in (the fifth root of q_prev above all) out of the dependent chain:
-// kw_prepare(q_prev, ...) followed by kw_solve(q_in, ...) performs exactly the operations of the
-// reference, in its order.
+// Split in two so that a routing loop can hoist everything that does not depend on the upstream
+// inflow q_in out of the dependent chain: the fifth root of q_prev above all, and the whole first
+// Newton update but for the "- C". kw_prepare(q_prev, ...) followed by kw_solve(q_in, ...) performs
+// the operations of the reference, in its order.
+//
+// Bound on the GPU: latency. One solve after another runs down a main stem, so what counts is the
+// length of the instruction stream of one solve, not its throughput: a dependent FP64 operation
+// takes 4.5 cycles, a branch on a vote about 60 and an IEEE division 70. The updates are therefore
+// straight code over all lanes (a lane that has converged keeps its value), with one vote after the
+// fourth and one after each further one, and they divide in range (wfh_div_by): 750 cycles for a
+// river solve, with the loop's branches and IEEE divisions about 2000.
 struct KwPrep {
-    double dt_dx;  // dt / dx
-    double u_prev; // q_prev^(1/5) (0 for negative q_prev)
-    double a_u3;   // alpha * u_prev * u_prev * u_prev
-    double lat;    // dt * q_lat
+    double dt_dx;   // dt / dx
+    double u_prev;  // q_prev^(1/5) (0 for negative q_prev)
+    double a_u3;    // alpha * u_prev * u_prev * u_prev
+    double lat;     // dt * q_lat
     double q_prev, q_lat;
+    double g0, df0, y0;  // first update from u_prev: f(u) + C, f'(u), 1 / f'(u) (wfh_rcp)
+    bool fast;           // u_prev > 0 and every quotient of the updates in range (kw_range_ok)
 };
 
-WFH_HD KwPrep kw_prepare(double q_prev, double q_lat, double alpha, double dt, double dx) {
+// f(u) + C and f'(u) of the kinematic wave in the fifth root u of the discharge
+WFH_HD void kw_terms(const double u, const double dt_dx, const double alpha, double& g, double& df) {
+    const double u2 = u * u;
+    const double u3 = u2 * u;
+    g = u3 * (dt_dx * u2 + alpha);
+    df = u2 * (5.0 * dt_dx * u2 + 3.0 * alpha);
+}
+
+// alpha, dt / dx and the previous discharge such that no term of the updates leaves the normal range
+// (kw_solve bounds C): u starts between 2^-100 and 2^100 and stays below 2^130 then, f and f' lie
+// between 2^-234 and 2^720, and a residual that is divided is above 1e-12.
+WFH_HD bool kw_range_ok(const double dt_dx, const double alpha) {
+    return alpha >= 0x1p-30 && alpha <= 0x1p60 && dt_dx >= 0x1p-30 && dt_dx <= 0x1p60;
+}
+
+// kw_prepare with dt / dx given, and whether kw_range_ok holds
+WFH_HD KwPrep kw_prepare_dx(double q_prev, double q_lat, double alpha, double dt, double dt_dx, bool range_ok) {
     KwPrep p;
-    p.dt_dx = dt / dx;
-    p.u_prev = q_prev >= 0.0 ? wfh_pow(q_prev, 0.2) : 0.0;
+    p.dt_dx = dt_dx;
+    const double root = wfh_pow(q_prev, 0.2);
+    p.u_prev = q_prev >= 0.0 ? root : 0.0;
     p.a_u3 = alpha * p.u_prev * p.u_prev * p.u_prev;
     p.lat = dt * q_lat;
     p.q_prev = q_prev;
     p.q_lat = q_lat;
+    kw_terms(p.u_prev, dt_dx, alpha, p.g0, p.df0);
+    p.y0 = wfh_rcp(p.df0);
+    p.fast = range_ok && q_prev >= 0x1p-498 && q_prev <= 0x1p498;
     return p;
 }
 
-WFH_HD void kw_solve(double q_in, const KwPrep& p, double alpha, double& q, double& area) {
-    if (q_in + p.q_prev + p.q_lat == 0.0) {
-        q = 0.0;
-        area = 0.0;
-        return;
-    }
-    const double dt_dx = p.dt_dx;
-    const double C = dt_dx * q_in + p.a_u3 + p.lat;
-    double u = p.u_prev > 0.0 ? p.u_prev : wfh_cbrt(C / alpha);
+WFH_HD KwPrep kw_prepare(double q_prev, double q_lat, double alpha, double dt, double dx) {
+    const double dt_dx = dt / dx;
+    return kw_prepare_dx(q_prev, q_lat, alpha, dt, dt_dx, kw_range_ok(dt_dx, alpha));
+}
+
+// The reference's loop as it stands, for operands out of range and for a start from C.
+//
+// The reference stops on |f| <= 1e-12 or after 3000 updates. For large C (|C| above about 1e4) the
+// rounding noise of f exceeds 1e-12, the test can never pass and the iteration settles on a fixed
+// point or a two-cycle of adjacent doubles until the limit. The update is a fixed function of u
+// (every other input is constant), so once a value repeats the rest of the sequence is known: the
+// value after update 3000 is taken from the cycle instead of running the remaining updates. Every
+// residual test the shortcut skips would have evaluated one of the cycle's values, all of which
+// already failed it.
+WFH_HD double kw_newton_any(double u, const double C, const double dt_dx, const double alpha) {
     const double c1 = 5.0 * dt_dx, c2 = 3.0 * alpha;
-    // The reference stops on |f| <= 1e-12 or after 3000 updates. For large C (|C| above about
-    // 1e4) the rounding noise of f exceeds 1e-12, the test can never pass and the iteration
-    // settles on a fixed point or a two-cycle of adjacent doubles until the limit. The update
-    // is a fixed function of u (every other input is constant), so once a value repeats the
-    // rest of the sequence is known: the value after update 3000 is taken from the cycle
-    // instead of running the remaining updates. Every residual test the shortcut skips would
-    // have evaluated one of the cycle's values, all of which already failed it.
     double u_pp = NaN_;  // the value two updates back
     for (int k = 0; k < 3000; ++k) {
         const double u2 = u * u;
@@ -284,10 +321,132 @@ WFH_HD void kw_solve(double q_in, const KwPrep& p, double alpha, double& q, doub
         }
         u_pp = u_c;
     }
-    u = wfh_max(u, WFH_KIN_WAVE_MIN_FLOW_QROOT);
+    return u;
+}
+
+// A solve on its way: u, the value before it, and f(u), f'(u) of a lane whose iteration goes on.
+struct KwRun {
+    double u, u_p, f, df;
+    bool live;  // not converged after the straight updates
+    bool any;   // not begun: a start from C, or operands out of range
+    bool zero;  // no flow at all
+};
+
+// The straight part of a solve: four updates. DRY: the cells of a wave are often all dry (overland
+// flow), which is worth a vote.
+template <bool DRY>
+WFH_HD KwRun kw_begin(double q_in, const KwPrep& p, double alpha) {
+    KwRun s;
+    const double dt_dx = p.dt_dx;
+    const double C = dt_dx * q_in + p.a_u3 + p.lat;
+    s.zero = q_in + p.q_prev + p.q_lat == 0.0;
+    s.u = s.u_p = s.f = s.df = 0.0;
+    s.live = s.any = false;
+    if (DRY && !WFH_ANY(!s.zero)) return s;
+    const bool ok = p.fast && wfh_fabs(C) <= 0x1p60;
+    s.any = !ok && !s.zero;
+    // First update: nothing of it depends on C but the residual.
+    double u = p.u_prev, g = p.g0, df = p.df0;
+    double f = g - C;
+    bool live = ok && !s.zero && !(wfh_fabs(f) <= 1.0e-12);
+    double v = u - wfh_div_by(f, df, p.y0);
+    v = v > 0.0 ? v : WFH_KIN_WAVE_MIN_FLOW_QROOT;  // also for NaN
+    double u_p = u;
+    u = live ? v : u;
+    // Three more without a vote: a river solve takes three to five updates.
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        kw_terms(u, dt_dx, alpha, g, df);
+        f = g - C;
+        live = live && !(wfh_fabs(f) <= 1.0e-12);
+        v = u - wfh_div_by(f, df, wfh_rcp(df));
+        v = v > 0.0 ? v : WFH_KIN_WAVE_MIN_FLOW_QROOT;
+        u_p = u;
+        u = live ? v : u;
+    }
+    kw_terms(u, dt_dx, alpha, g, df);
+    f = g - C;
+    s.live = live && !(wfh_fabs(f) <= 1.0e-12);
+    s.u = u, s.u_p = u_p, s.f = f, s.df = df;
+    return s;
+}
+
+// The rest of it, for the lanes with live or any set.
+//
+// A cell whose previous flow is KIN_WAVE_MIN_FLOW starts at u = 1e-6, jumps to about 1e11 and comes
+// down by a fifth per update, about 126 of them. While f(u) + C is above 1024 |C| + 1e-8 the next
+// four updates need no test: an update takes between a tenth and a half off u (f is at least half
+// of f + C, f' at most five and at least three times (f + C) / u), so that f + C falls by less than
+// 7.6-fold in each and every residual stays above |C| + 1e-11, no value repeats and none is
+// negative. They run as four bare updates per vote, 95 cycles each instead of 200.
+WFH_HD void kw_end(double q_in, const KwPrep& p, double alpha, KwRun& s) {
+    const double dt_dx = p.dt_dx;
+    const double C = dt_dx * q_in + p.a_u3 + p.lat;
+    double u = s.u, u_p = s.u_p, f = s.f, df = s.df, g;
+    bool live = s.live;
+    int n = 5;  // u is iterate n - 1
+    if (s.any) {
+        u = p.u_prev > 0.0 ? p.u_prev : wfh_cbrt(C / alpha);
+        if (kw_range_ok(dt_dx, alpha) && wfh_fabs(C) <= 0x1p60 && wfh_fabs(u) >= 0x1p-100 && wfh_fabs(u) <= 0x1p100) {
+            n = 1;
+            u_p = NaN_;
+            kw_terms(u, dt_dx, alpha, g, df);
+            f = g - C;
+            live = !(wfh_fabs(f) <= 1.0e-12);
+        } else {
+            u = kw_newton_any(u, C, dt_dx, alpha);
+        }
+    }
+    const double far = 1024.0 * wfh_fabs(C) + 1.0e-8;
+    bool fall = live && f + C > far;
+    while (WFH_ANY(fall)) {
+        double v = u, w = u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            kw_terms(v, dt_dx, alpha, g, df);
+            w = v;
+            v = v - wfh_div_by(g - C, df, wfh_rcp(df));
+        }
+        kw_terms(v, dt_dx, alpha, g, df);
+        u_p = fall ? w : u_p;
+        u = fall ? v : u;
+        n = fall ? n + 4 : n;
+        fall = fall && g > far;
+    }
+    kw_terms(u, dt_dx, alpha, g, df);
+    f = g - C;
+    live = live && !(wfh_fabs(f) <= 1.0e-12);
+    // The end of the sequence is watched (kw_newton_any): a fixed point or a two-cycle entered in the
+    // straight part is found here just as well, since it goes on.
+    for (; WFH_ANY(live); ++n) {
+        double v = u - wfh_div_by(f, df, wfh_rcp(df));
+        v = v > 0.0 ? v : WFH_KIN_WAVE_MIN_FLOW_QROOT;
+        const bool cycle = v == u_p;
+        const bool end = v == u || cycle || n >= 3000;
+        u_p = live ? u : u_p;
+        u = live && !(cycle && ((3000 - n) & 1) && v != u) ? v : u;
+        kw_terms(u, dt_dx, alpha, g, df);
+        f = g - C;
+        live = live && !end && !(wfh_fabs(f) <= 1.0e-12);
+    }
+    s.u = u;
+    s.live = s.any = false;
+}
+
+WFH_HD void kw_result(const KwRun& s, double alpha, double& q, double& area) {
+    const double u = s.zero ? 0.0 : wfh_max(s.u, WFH_KIN_WAVE_MIN_FLOW_QROOT);
     const double u3 = u * u * u;
     q = u3 * u * u;
-    area = alpha * u3;
+    area = s.zero ? 0.0 : alpha * u3;
+}
+
+template <bool DRY = false>
+WFH_HD void kw_solve(double q_in, const KwPrep& p, double alpha, double& q, double& area) {
+    KwRun s = kw_begin<DRY>(q_in, p, alpha);
+    if (WFH_ANY(s.live || s.any)) {
+        if (s.live || s.any) kw_end(q_in, p, alpha, s);
+    }
+    kw_result(s, alpha, q, area);
 }
 
 // The Newton iteration of kw_solve from the start u (the same updates, stopping rule and cycle
@@ -416,7 +575,7 @@ struct Column {
 
 // water_table_change  Wflow/src/utils.jl:1090-1131
 template <int N>
-WFH_HD void water_table_change(const Column<N>& s, double net_flux, double sy, double dt, double& dh, double& exf) {
+WFH_HD_INLINE void water_table_change(const Column<N>& s, double net_flux, double sy, double dt, double& dh, double& exf) {
     if (net_flux <= 0.0) {
         dh = net_flux * dt / sy;
     } else {
@@ -441,7 +600,7 @@ WFH_HD void water_table_change(const Column<N>& s, double net_flux, double sy, d
 
 // update_ustorelayerdepth!(soil, zi_prev, water_table_depth, i)  Wflow/src/soil/soil.jl:1213-1259
 template <int N>
-WFH_HD void update_ustorelayerdepth(Column<N>& s, double zi_prev, double zi) {
+WFH_HD_INLINE void update_ustorelayerdepth(Column<N>& s, double zi_prev, double zi) {
     const int nprev = s.n_unsat;
     double t[N];
     const int nnew = set_layerthickness<N>(zi, s.cum, s.act, t);
@@ -480,7 +639,7 @@ WFH_HD void update_ustorelayerdepth(Column<N>& s, double zi_prev, double zi) {
 // remainder of the solve reads) and the function returns true; the caller must apply it before
 // the column is read again. The sub-stepped branch always updates the column itself.
 template <int N>
-WFH_HD bool kinematic_wave_ssf(double q_in, double q_prev, double zi_prev, double q_net, double slope, double sy,
+WFH_HD_INLINE bool kinematic_wave_ssf(double q_in, double q_prev, double zi_prev, double q_net, double slope, double sy,
                                double d, double dt, double dx, double dw, double q_max, double kh0, double f,
                                double z_exp, const SsfPrep& pp, Column<N>& soil, const bool defer_update, double& q_out,
                                double& zi_out, double& exf_out, double& net_out) {
@@ -552,6 +711,96 @@ WFH_HD bool kinematic_wave_ssf(double q_in, double q_prev, double zi_prev, doubl
     exf_out = exf;
     net_out = net;
     return deferred;
+}
+
+// One subsurface solve (kinematic_wave_ssf, single-step branch) with everything that does not
+// depend on the upstream inflow formed beforehand: the divisors' reciprocals (wfh_rcp) and, of the
+// bottom unsaturated layer, which takes the rise of the water table unless it fills, the capacity
+// and the drainable porosity. What is left for the moment the inflow arrives are some 40 dependent
+// operations and five in-range quotients, against eight IEEE divisions of 70 cycles each. The
+// operations and their order are kinematic_wave_ssf's; operands out of range, a third Newton update, a
+// layer that fills and a water table that falls below the soil or moves so far that it needs
+// sub-steps are left to it, so that the whole solve holds a single vote.
+struct SsfQuick {
+    double y_df;              // 1 / (dt / dx + 1 / celerity)
+    double qcap;              // q_max * dw
+    double wa, y_wa;          // dw * dx
+    double y_sy;
+    double cap, thick, syd, y_syd;  // bottom unsaturated layer: capacity / dt, thickness, porosity
+    int n_unsat;
+    bool ok;
+};
+
+WFH_HD bool ssf_divisor_ok(const double x) { return x >= 0x1p-100 && x <= 0x1p100; }
+WFH_HD bool ssf_value_ok(const double x) {
+    const double a = wfh_fabs(x);
+    return a == 0.0 || (a >= 0x1p-400 && a <= 0x1p100);
+}
+
+template <int N>
+WFH_HD SsfQuick ssf_quick_prepare(double q_prev, double zi_prev, double q_net, double sy, double d, double dt,
+                                  double dx, double dw, double q_max, const SsfPrep& pp, const Column<N>& soil) {
+    SsfQuick k;
+    k.y_df = wfh_rcp(pp.df);
+    k.qcap = q_max * dw;
+    k.wa = dw * dx;
+    k.y_wa = wfh_rcp(k.wa);
+    k.y_sy = wfh_rcp(sy);
+    double us = 0.0, th = 0.0;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (j == soil.n_unsat - 1) {
+            us = soil.ustore[j];
+            th = soil.thick[j];
+        }
+    k.n_unsat = soil.n_unsat;
+    k.cap = wfh_max(th * soil.theta_e - us, 0.0) / dt;
+    k.thick = th;
+    k.syd = soil.theta_e - (us / th);
+    k.y_syd = wfh_rcp(k.syd);
+    k.ok = ssf_divisor_ok(pp.df) && ssf_divisor_ok(pp.dt_dx) && ssf_divisor_ok(pp.cinv) && ssf_divisor_ok(k.wa) &&
+           ssf_divisor_ok(sy) && ssf_divisor_ok(dt) && ssf_value_ok(q_prev) && ssf_value_ok(pp.qp_cel) &&
+           ssf_value_ok(q_net) && ssf_value_ok(zi_prev) && ssf_value_ok(d) && ssf_value_ok(k.qcap) &&
+           (k.n_unsat == 0 || (ssf_value_ok(k.cap) && (k.cap == 0.0 || ssf_divisor_ok(k.syd))));
+    return k;
+}
+
+// False when the solve is one for kinematic_wave_ssf; otherwise its results, with the column's
+// update_ustorelayerdepth!(soil, zi_prev, zi_out) left to the caller when `deferred` is set.
+WFH_HD bool ssf_quick_solve(double q_in, double q_prev, double zi_prev, double q_net, double sy, double d, double dt,
+                            const SsfPrep& pp, const SsfQuick& k, double& q_out, double& zi_out, double& exf_out,
+                            double& net_out, bool& deferred) {
+    const bool dry = q_in + q_prev == 0.0 && q_net <= 0.0;
+    // Newton on a linear equation: the second update's residual is rounding
+    const double C = pp.dt_dx * (q_in + q_net) + pp.qp_cel;
+    const double q0 = (q_prev + q_in) / 2.0;
+    const double r0 = pp.dt_dx * q0 + pp.cinv * q0 - C;
+    const double q1 = __builtin_fmax(q0 - wfh_div_by(r0, pp.df, k.y_df), WFH_KIN_WAVE_MIN_FLOW);
+    const double r1 = pp.dt_dx * q1 + pp.cinv * q1 - C;
+    const double q2 = __builtin_fmax(q1 - wfh_div_by(r1, pp.df, k.y_df), WFH_KIN_WAVE_MIN_FLOW);
+    double q = wfh_fabs(r0) <= 1.0e-12 ? q1 : q2;
+    bool ok = k.ok && ssf_value_ok(q_in) && wfh_fabs(r1) <= 1.0e-12;
+    q = __builtin_fmin(q, k.qcap);
+    const double net = wfh_div_by(q_in + q_net - q, k.wa, k.y_wa);
+    // water_table_change
+    const bool up = net > 0.0;
+    const bool part = net < k.cap;
+    const double dh_up = part ? wfh_div_by(net * dt, k.syd, k.y_syd) : k.thick;
+    const double dh_dn = wfh_div_by(net * dt, sy, k.y_sy);
+    const bool layer = up && k.n_unsat > 0;
+    const double dh = layer ? dh_up : (up ? 0.0 : dh_dn);
+    const double exf = up && !layer ? net : 0.0;
+    ok = ok && (part || !layer);  // (the layer fills, about one solve in a hundred)
+    double zi = zi_prev - dh;
+    ok = ok && !(zi > d);  // (water that leaves no room below: the excess lowers q)
+    zi = wfh_clamp(zi, 0.0, d);
+    ok = ok && wfh_fabs(zi - zi_prev) <= 0.0998;
+    q_out = dry ? 0.0 : q;
+    zi_out = dry ? d : zi;
+    exf_out = dry ? 0.0 : exf;
+    net_out = dry ? 0.0 : net;
+    deferred = !dry;
+    return ok || dry;
 }
 
 }  // namespace wfh

@@ -146,9 +146,10 @@ struct Dev {
     const double* res_rce;     // [nres] free weir rating curve exponent
     int* abort_flag;           // the routing kernels' abort flag (RouteArgs::abort_flag)
     int* nonfinite_flag;       // set by the vertical kernel when a cell's forcing is not finite
-    const int* chain_land;     // [nchunks] 1: a chain chunk of the land lists (see run_chain)
-    const int* chain_rl;       // [nchunks] 1: all 64 cells are river cells and a chain of the river lists
-    const int* chain_sup;      // [nchunks] 1: a chain chunk of the snow transport's lists (sup_ptr)
+    // the passes of each chunk's schedule (run_sched, chunk_ranks): every cell's rank in its chunk
+    // and the chunk's number of ranks, over all cells and over its river cells
+    const uint8_t *rank_land, *rank_riv;     // [n]
+    const uint8_t *nrank_land, *nrank_riv;   // [nchunks]
     int res_linked;            // some free weir is linked to a lower reservoir
     const int *res_lower, *res_upper;  // [nres] linked lower / upper reservoir, or -1
     uint64_t* res_xfer;        // [nres] single-consumer slot: the linked free weir's reverse flow of
@@ -221,7 +222,7 @@ struct AdArgs {
     const int* rp_node;    // [nriv] node of the river cell at each river position
     const int *fp_sup_ptr, *fp_sup_idx;  // [nriv+1], [Er]: all upstream river positions, in the
                                          // order of the reference's river topological sort
-    const int* chain_r;    // [nchunks_r] 1: a chain chunk (see run_chain)
+    const uint8_t *rank_r, *nrank_r;  // [nriv], [nchunks_r]: schedule of the river positions (run_sched)
     int nchunks_r;
 };
 
@@ -402,188 +403,272 @@ __device__ __forceinline__ void fold_in(double& acc1, double& acc2, double q, do
 }
 
 // One family of routing sub-steps (all subsurface, all overland or all river sub-steps of the
-// model step) for the 64 cells of a wave. Every lane runs the same code; the wave advances a
-// diagonal wavefront over (cell, sub-step): a lane computes sub-step k once all upstream cells
-// have produced their sub-step-k outflow and, for multi-step families, its in-wave downstream
-// cell has computed sub-step k-1 (so the outflow it is about to replace has been used).
+// model step) for the 64 cells of a wave, as a sequence of passes in which the lanes of the pass
+// compute one sub-step each.
 //
-// In-wave exchange goes through a 64-entry table in LDS: each round every lane writes its
-// (next sub-step, last outflow) pair, then reads the entries of its in-wave upstream cells with
-// independent loads and keeps the values that belong to its current sub-step. Outflow to a
-// consumer in another wave goes through that consumer's global slot (one per edge and
-// sub-step); such slots are polled once per round and picked up in the next round, so the poll
-// latency overlaps the round's work. The upstream outflow is folded in ascending edge order,
-// the reference's sum_at order, as far as it has arrived. Returns false when the wave has to
+// Bound: the latency of one pass times the cells of the longest path, and in a pass the number of
+// instructions (4.5 cycles each, dependent or not) and of branches on votes (about 60 cycles). A
+// pass therefore holds little but what the next cell waits for: the inflow of the lane's sub-step
+// is read from LDS in one round trip (an in-wave upstream cell's outflow from the wave's table, an
+// outflow from another wave from this lane's inbox, a zero for an edge that is not there, at
+// addresses fixed beforehand), folded in ascending edge order (the reference's sum_at order), solved
+// (`compute`), published and written to the table; lanes whose solve turns out long follow
+// (`finish`), then the sums and the preparation of the next sub-step (`after`).
+//   One sub-step: a lane computes as soon as its inflow is there. Which in-wave cells are left is
+// one wave-uniform bit mask, held against each lane's mask of in-wave upstream cells, so a lane
+// that waits for a late inflow holds up nobody else.
+//   Several sub-steps: a fixed schedule. `rank` is the cell's place in its chunk (chunk_ranks), an
+// in-wave upstream cell having the next lower rank, and in pass t a lane computes sub-step
+// t - rank: the sub-steps of a chain run as a diagonal, and the lanes of a wave stay in step.
+//   Once the inflow from other waves is complete, either kind runs its remaining passes in the
+// order of the ranks, without a vote: 260 cycles a pass (trivial solve) instead of 950.
+//
+// Outflow to a consumer in another wave goes through that consumer's global slot (one per edge
+// and sub-step, cleared by the consumer). Slots are polled for all lanes of the wave together, at
+// most RING sub-steps ahead, when a pass lacks one (or, overlapped with the pass, when a lane of
+// the next passes does), and taken into the inbox; so a wave that waits for its main stem has the
+// inflow of its tributaries before the main stem arrives. A wave waits only for chunks of smaller
+// index, so the ticket order keeps the launch free of deadlock. Returns false when the wave has to
 // stop (a wait exceeded its limit, or another wave raised the abort flag).
-template <int FOLD, class Compute>
-__device__ __forceinline__ bool run_family(const RouteArgs& a, const int lane, const int c, const bool part,
-                                           const int S, const int* __restrict__ up_node,
-                                           const int* __restrict__ up_slot, const double* __restrict__ up_f,
-                                           const int e0, const int e1, uint64_t* slots, const size_t stride,
-                                           const int my_slot, const bool pub_cross, const int cons_lane,
-                                           int* lds_k, double* lds_q, Compute& compute, const double acc0 = 0.0) {
-    // The first PF upstream edges are buffered in registers; further edges (a cell with more
-    // than PF upstream cells) are taken one per round in order, after the buffered ones.
-    constexpr int PF = 4;
-    int k = part ? 0 : S;
-    int e = e0;
-    double acc1 = acc0, acc2 = 0.0, qv = 0.0;  // acc0: start of the first sub-step's fold
-    const int npf = (e1 - e0) < PF ? (e1 - e0) : PF;
-    int en[PF], es[PF];
-    double ef[PF], buf[PF];
-    uint64_t v[PF];
-    bool pol[PF];
-    // Every lane loads PF entries (unused ones at a valid index); the empty asm takes them all as
-    // operands, so the compiler issues the loads together and waits once, instead of moving each
-    // into the per-lane branch that uses it and waiting for them one by one.
-    int un[PF], us[PF];
-    double uf[PF];
-#pragma unroll
-    for (int j = 0; j < PF; ++j) {
-        const int ej = j < npf ? e0 + j : (npf > 0 ? e0 : 0);
-        un[j] = up_node[ej];
-        us[j] = up_slot[ej];
-        uf[j] = (FOLD != FOLD_RIV && FOLD != FOLD_SNOW) ? up_f[ej] : 0.0;
-    }
-    static_assert(PF == 4, "the operand list below names four edges");
-    asm volatile("" : "+v"(un[0]), "+v"(un[1]), "+v"(un[2]), "+v"(un[3]), "+v"(us[0]), "+v"(us[1]), "+v"(us[2]),
-                 "+v"(us[3]), "+v"(uf[0]), "+v"(uf[1]), "+v"(uf[2]), "+v"(uf[3]));
-#pragma unroll
-    for (int j = 0; j < PF; ++j) {
-        const bool use = j < npf;
-        en[j] = use ? un[j] : c * WAVE;
-        es[j] = use ? us[j] : 0;
-        ef[j] = use ? uf[j] : 0.0;
-        buf[j] = 0.0;
-        v[j] = SLOT_EMPTY;
-        pol[j] = false;
-    }
-    unsigned have = 0;  // bit j: buf[j] holds edge e0 + j's outflow for sub-step k
-    long spin = 0;
-    while (__any(k < S)) {
-        bool act = k < S;
-        // (1) publish this lane's state to the wave's table
-        lds_k[lane] = k;
-        lds_q[lane] = qv;
-        __builtin_amdgcn_wave_barrier();
-        // (2) pick up last round's polls; gather the in-wave upstream outflow that is ready. The
-        // table entries of all PF producers are read unconditionally (unused edges point at
-        // lane 0), so the reads overlap and one wait covers them.
-        int tk[PF];
-        double tq[PF];
+//
+// The exchange before this one compared (sub-step, outflow) pairs of the upstream cells in every
+// pass and let each lane compute whenever it was ready; the lanes of a wave drifted apart until each
+// sub-step of each cell took a pass of its own. With it and the solves of that time an hourly step
+// took 0.56 ms on 61 x 67 cells, 2.43 ms on 509 x 487 and 18.1 ms on 4096 x 4096, a daily one (24
+// land and 96 river sub-steps) 14.6 ms on 256 x 256; now 0.30, 1.68, 15.7 and 2.0 ms.
+constexpr int SCHED_PF = 4;                             // upstream edges with a place in the inbox
+constexpr int SCHED_ZERO = (SCHED_PF + 1) * WAVE;       // a zero after the table row and the inbox rows
+constexpr int SCHED_ROWS = SCHED_ZERO + 8;              // doubles of one sub-step
+constexpr int SCHED_RING = 4;                           // sub-steps the inbox holds
+
+// The abort flag as a wave-uniform value (a branch on the value a lane loaded is a per-lane one)
+__device__ __forceinline__ bool aborted(const RouteArgs& a) {
+    return __builtin_amdgcn_readfirstlane(
+               __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+}
+// The next ticket, the same for all lanes and known to be so (a shuffle's result is not)
+__device__ __forceinline__ unsigned long long next_ticket(unsigned long long* counter, const int lane) {
+    unsigned long long t = 0;
+    if (lane == 0) t = atomicAdd(counter, 1ull);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)(unsigned)t);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((int)(unsigned)(t >> 32));
+    return (unsigned long long)hi << 32 | lo;
+}
+
+// for the families' lambdas, which run_sched calls at two places
+#define ROUTE_INLINE __attribute__((always_inline))
+
+template <int RING>
+__device__ __forceinline__ void sched_init(double* lds, const int lane) {
+    if (lane < RING) lds[lane * SCHED_ROWS + SCHED_ZERO] = 0.0;
+}
+
+template <int FOLD, int RING, class Compute, class Finish, class After>
+__device__ __forceinline__ bool run_sched(const RouteArgs& a, const int lane, const int c, const bool part,
+                                          const int S, const int rank, const int nrank,
+                                          const int* __restrict__ up_node, const int* __restrict__ up_slot,
+                                          const double* __restrict__ up_f, const int e0, const int e1, uint64_t* slots,
+                                          const size_t stride, const int my_slot, const bool pub_cross, double* lds,
+                                          Compute& compute, const Finish& finish, const After& after,
+                                          const double acc0 = 0.0) {
+    constexpr int PF = SCHED_PF;
+    static_assert((RING & (RING - 1)) == 0, "sub-step k uses row k mod RING");
+    constexpr bool FRAC = FOLD != FOLD_RIV && FOLD != FOLD_SNOW;
+    const int ne = part ? e1 - e0 : 0;
+    int at[PF], es[PF];
+    double ef[PF];
+    unsigned ext = 0;   // bit j: edge e0 + j comes from another wave
+    uint64_t need = 0;  // in-wave upstream lanes (used with one sub-step)
+    {
+        // Every lane loads PF entries (unused ones at a valid index); the empty asm takes them all
+        // as operands, so the compiler issues the loads together and waits once, instead of moving
+        // each into the per-lane branch that uses it and waiting for them one by one.
+        int un[PF], us[PF];
+        double uf[PF];
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
-            tk[j] = lds_k[en[j] & (WAVE - 1)];
-            tq[j] = lds_q[en[j] & (WAVE - 1)];
+            const int ej = j < ne ? e0 + j : (ne > 0 ? e0 : 0);
+            un[j] = up_node[ej];
+            us[j] = up_slot[ej];
+            uf[j] = FRAC ? up_f[ej] : 0.0;
         }
-        bool got = false;
+        static_assert(PF == 4, "the operand list below names four edges");
+        asm volatile("" : "+v"(un[0]), "+v"(un[1]), "+v"(un[2]), "+v"(un[3]), "+v"(us[0]), "+v"(us[1]), "+v"(us[2]),
+                     "+v"(us[3]), "+v"(uf[0]), "+v"(uf[1]), "+v"(uf[2]), "+v"(uf[3]));
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
-            const bool from_slot = pol[j] && v[j] != SLOT_EMPTY;
-            if (from_slot)
-                __hip_atomic_store(slots + (size_t)k * stride + es[j], SLOT_EMPTY, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            const bool from_wave = act && j < npf && (en[j] >> 6) == c && !(have & (1u << j)) && tk[j] == k + 1;
-            buf[j] = from_slot ? wfh_from_bits(v[j]) : (from_wave ? tq[j] : buf[j]);
-            have |= (from_slot || from_wave) ? (1u << j) : 0u;
-            got = got || from_slot || from_wave;
+            const bool use = j < ne, in = (un[j] >> 6) == c;
+            at[j] = !use ? SCHED_ZERO : in ? (un[j] & (WAVE - 1)) : (1 + j) * WAVE + lane;
+            es[j] = us[j];
+            ef[j] = use ? uf[j] : 0.0;
+            ext |= (use && !in) ? (1u << j) : 0u;
+            need |= (use && in) ? 1ull << (un[j] & (WAVE - 1)) : 0ull;
         }
-        // (3) issue this round's polls for the cross-wave edges still missing
+    }
+    const bool many = __any(ne > PF);  // wave-uniform
+    if (many)
+        for (int e = e0 + PF; e < e0 + ne; ++e) {
+            const int u = up_node[e];
+            need |= (u >> 6) == c ? 1ull << (u & (WAVE - 1)) : 0ull;
+        }
+    int kf = ext ? 0 : S;  // sub-steps of this lane whose inflow from other waves is in the inbox
+    unsigned got = 0;      // bit j: edge e0 + j of sub-step kf has arrived
+    uint64_t v[PF];        // the poll in flight
+    const auto fetch = [&](const bool want) {
+        const unsigned miss = want ? ext & ~got : 0u;
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
-            pol[j] = act && j < npf && (en[j] >> 6) != c && !(have & (1u << j));
             v[j] = SLOT_EMPTY;
-            if (pol[j])
-                v[j] = __hip_atomic_load(slots + (size_t)k * stride + es[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (miss >> j & 1u)
+                v[j] = __hip_atomic_load(slots + (size_t)kf * stride + es[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        // (4) fold the buffered prefix in edge order, then at most one further edge
-        if (act) {
+        __builtin_amdgcn_wave_barrier();  // (see the loop)
+    };
+    bool complete = !__any(kf < S);  // all inflow from other waves is in the inbox (wave-uniform)
+    const auto collect = [&]() -> bool {  // true when something arrived
+        bool in[PF], any = false;
 #pragma unroll
-            for (int j = 0; j < PF; ++j)
-                if (e == e0 + j && (have & (1u << j))) {
-                    fold_in<FOLD>(acc1, acc2, buf[j], ef[j]);
-                    ++e;
-                }
-            if (e >= e0 + PF && e < e1) {
-                const int u = up_node[e];
-                const double f = (FOLD != FOLD_RIV && FOLD != FOLD_SNOW) ? up_f[e] : 0.0;
-                double q = 0.0;
-                bool took = false;
-                if ((u >> 6) == c) {
-                    if (lds_k[u & (WAVE - 1)] == k + 1) {
-                        q = lds_q[u & (WAVE - 1)];
-                        took = true;
-                    }
-                } else {
-                    took = slot_take(slots + (size_t)k * stride + up_slot[e], q);
-                }
-                if (took) {
-                    fold_in<FOLD>(acc1, acc2, q, f);
-                    ++e;
-                    got = true;
-                }
-            }
+        for (int j = 0; j < PF; ++j) {
+            in[j] = v[j] != SLOT_EMPTY;
+            any = any || in[j];
         }
-        // (5) compute the ready lanes. Lanes whose in-wave upstream cells complete here are
-        // served within the same round: the producers republish, the consumers gather, fold and
-        // compute in turn, so a chain inside the wave advances several cells per round. Every
-        // pass computes at least one sub-step, so the passes end.
-        bool any_done = false;
-        for (int pass = 0; pass < WAVE * S; ++pass) {
-            const int kcons = lds_k[cons_lane & (WAVE - 1)];
-            const bool bp = S == 1 || cons_lane < 0 || kcons >= k;
-            const bool can = act && e == e1 && bp;
-            __builtin_amdgcn_wave_barrier();
-            if (!__any(can)) break;
-            any_done = true;
-            if (can) {
-                qv = compute(k, acc1, acc2);
-                if (pub_cross) slot_put(slots + (size_t)k * stride + my_slot, qv);
-                ++k;
-                e = e0;
-                acc1 = 0.0;
-                acc2 = 0.0;
-                have = 0;
-            }
-            act = k < S;
-            lds_k[lane] = k;
-            lds_q[lane] = qv;
-            __builtin_amdgcn_wave_barrier();
+        if (!__any(any)) return false;
 #pragma unroll
-            for (int j = 0; j < PF; ++j) {
-                tk[j] = lds_k[en[j] & (WAVE - 1)];
-                tq[j] = lds_q[en[j] & (WAVE - 1)];
+        for (int j = 0; j < PF; ++j)
+            if (in[j]) {
+                __hip_atomic_store(slots + (size_t)kf * stride + es[j], SLOT_EMPTY, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+                lds[(kf & (RING - 1)) * SCHED_ROWS + (1 + j) * WAVE + lane] = wfh_from_bits(v[j]);
+                got |= 1u << j;
             }
-#pragma unroll
-            for (int j = 0; j < PF; ++j) {
-                const bool from_wave =
-                    act && j < npf && (en[j] >> 6) == c && !(have & (1u << j)) && tk[j] == k + 1;
-                buf[j] = from_wave ? tq[j] : buf[j];
-                have |= from_wave ? (1u << j) : 0u;
-            }
-            if (act) {
-#pragma unroll
-                for (int j = 0; j < PF; ++j)
-                    if (e == e0 + j && (have & (1u << j))) {
-                        fold_in<FOLD>(acc1, acc2, buf[j], ef[j]);
-                        ++e;
-                    }
+        __builtin_amdgcn_wave_barrier();  // (see the loop)
+        const bool full = kf < S && got == ext;
+        kf = full ? kf + 1 : kf;
+        got = full ? 0u : got;
+        complete = !__any(kf < S);
+        return true;
+    };
+    // A pass of the lanes that execute: inflow, solve, publish. The lanes whose solve does not end in
+    // its straight part publish after the others (`finish`), so that a long solve (an overland one
+    // can take 126 updates) does not hold up the cells below the other lanes.
+    const auto pass = [&](const int k, double acc1, double acc2) ROUTE_INLINE {
+        double* const out = lds + (k & (RING - 1)) * SCHED_ROWS + lane;
+        uint64_t* const slot = slots + (size_t)k * stride + my_slot;
+        bool open = false;
+        const double q1 = compute(k, acc1, acc2, open);
+        if (!open) {
+            *out = q1;
+            if (pub_cross) slot_put(slot, q1);
+        }
+        if (__any(open)) {
+            if (open) {
+                const double q2 = finish(k);
+                *out = q2;
+                if (pub_cross) slot_put(slot, q2);
             }
         }
-        if (any_done || __any(got)) {
-            spin = 0;
+        after(k);
+    };
+    const int T = nrank > 0 ? nrank + S - 1 : 0;
+    uint64_t left = __ballot(part);  // one sub-step: lanes that have not computed
+    int mine = part ? rank : -S;     // this lane's first pass; -S once it has computed its only sub-step
+    int t = 0;
+
+    // ---- some inflow from other waves is still to come ----
+    // The per-lane branches of a poll, of a look at its values and of a pass are each closed by a wave
+    // barrier (no instruction): the compiler would else merge their ends with the ways round them, and
+    // take every wave-uniform variable that has two values there for a per-lane one, that is, keep
+    // the whole loop's state in vector registers and its branches under execution masks (1250 cycles
+    // for a pass with a trivial solve, where the scheduled passes below take 260).
+    // A poll issued beside a pass is looked at PASSES_PER_POLL passes later, when its values are
+    // there, so that no pass waits for memory.
+    constexpr int PASSES_PER_POLL = 2;
+    int pending = 0;  // passes until the poll in flight is looked at (0: none)
+    long spin = 0;
+    while (!complete || many) {
+        bool act, go;  // lanes of the pass; whether there is one (else the wave waits)
+        int k = 0;
+        if (S > 1) {
+            if (t >= T) break;
+            k = t - mine;
+            act = (unsigned)k < (unsigned)S;
+            go = !__any(act && kf <= k);
         } else {
-            __builtin_amdgcn_s_sleep(1);
+            if (left == 0) break;
+            act = mine >= 0 && kf > 0 && !(need & left);
+            go = __any(act);
+            left &= ~__ballot(act);
+            mine = act ? -1 : mine;
+        }
+        // polls: inflow that this pass lacks, or that the next passes do
+        const int kring = (k > 0 ? k : 0) + RING;  // inbox rows before this one are free or filled
+        const bool want = kf < S && kf < kring;
+        const bool soon = S > 1 ? kf <= k + PASSES_PER_POLL : mine >= 0 && !(need & left);
+        if (pending == 0 && (!go || __any(want && soon))) {
+            fetch(want);
+            pending = PASSES_PER_POLL + 1;
+        }
+        bool stop = false;
+        __builtin_amdgcn_wave_barrier();
+        if (act && go) {
+            const double* const row = lds + (k & (RING - 1)) * SCHED_ROWS;
+            double acc1 = acc0, acc2 = 0.0;
+#pragma unroll
+            for (int j = 0; j < PF; ++j) fold_in<FOLD>(acc1, acc2, row[at[j]], ef[j]);
+            for (int e = e0 + PF; e < e0 + ne; ++e) {
+                const int u = up_node[e];
+                const double f = FRAC ? up_f[e] : 0.0;
+                double qe = row[u & (WAVE - 1)];
+                if ((u >> 6) != c) {
+                    uint64_t* const sl = slots + (size_t)k * stride + up_slot[e];
+                    for (long w = 0; !stop && !slot_take(sl, qe); ++w) {
+                        __builtin_amdgcn_s_sleep(1);
+                        stop = w > a.spin_limit ||
+                               ((w & 255) == 255 &&
+                                __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                    }
+                }
+                fold_in<FOLD>(acc1, acc2, qe, f);
+            }
+            pass(k, acc1, acc2);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (many && __any(stop)) {  // (wave-uniform)
+            __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+        t += go && S > 1 ? 1 : 0;
+        pending -= pending > 0 ? 1 : 0;
+        if (!complete && (!go || pending == 1)) {
+            pending = 0;
+            if (collect()) spin = -1;
+        }
+        if (!go) {
             ++spin;
-            if ((spin & 255) == 0 && __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                return false;
+            if ((spin & 255) == 255 && aborted(a)) return false;
             if (spin > a.spin_limit) {
                 __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return false;
             }
+        } else {
+            spin = 0;
         }
     }
-    __builtin_amdgcn_wave_barrier();
+    if (many) return true;
+
+    // ---- all inflow from other waves is in the inbox: the passes left, in the order of the ranks ----
+    for (; t < T; ++t) {
+        const int k = t - mine;
+        if ((unsigned)k < (unsigned)S) {
+            const double* const row = lds + (k & (RING - 1)) * SCHED_ROWS;
+            double acc1 = acc0, acc2 = 0.0;
+            // an edge that is not there adds 0 (sums that start from 0 are never -0, so that is exact)
+#pragma unroll
+            for (int j = 0; j < PF; ++j) fold_in<FOLD>(acc1, acc2, row[at[j]], ef[j]);
+            pass(k, acc1, acc2);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
     return true;
 }
 
@@ -606,148 +691,6 @@ __device__ __forceinline__ bool wait_chunks(const RouteArgs& a, const int ca, co
         }
     }
     asm volatile("" ::: "memory");
-    return true;
-}
-
-__device__ __forceinline__ double readlane_f64(const double v, const int l) {
-    const uint64_t b = wfh_bits(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
-    return wfh_from_bits(((uint64_t)hi << 32) | lo);
-}
-
-// A family of one sub-step over a chain chunk: all 64 lanes valid, at most 4 upstream cells
-// each, and lane l's only upstream cell inside the chunk is lane l-1 (checked on the host). The
-// lanes first take their inflow from other chunks; then the lanes fold and solve one after the
-// other, each handing its outflow to the next through a register broadcast. The folds, in edge
-// order, and the solves are those of run_family, so the results are the same; what goes is the
-// per-hop exchange through LDS and the wave votes of run_family's in-round passes.
-template <int FOLD, class Compute>
-__device__ __forceinline__ bool run_chain(const RouteArgs& a, const int lane, const int c,
-                                          const int* __restrict__ up_node, const int* __restrict__ up_slot,
-                                          const double* __restrict__ up_f, const int e0, const int e1,
-                                          uint64_t* slots, const int my_slot, const bool pub_cross, Compute& compute,
-                                          const double acc0 = 0.0) {
-    constexpr int PF = 4;
-    const int ne = e1 - e0;
-    int en[PF], es[PF];
-    double ef[PF], buf[PF];
-    bool have[PF];
-#pragma unroll
-    for (int j = 0; j < PF; ++j) {
-        const bool use = j < ne;
-        const int ej = use ? e0 + j : (ne > 0 ? e0 : 0);  // (edge arrays hold at least one entry)
-        en[j] = use ? up_node[ej] : c * WAVE;
-        es[j] = use ? up_slot[ej] : 0;
-        ef[j] = (use && FOLD != FOLD_RIV && FOLD != FOLD_SNOW) ? up_f[ej] : 0.0;
-        buf[j] = 0.0;
-        have[j] = !use || (en[j] >> 6) == c;
-    }
-    long spin = 0;
-    for (;;) {
-        bool missing = false;
-#pragma unroll
-        for (int j = 0; j < PF; ++j) {
-            if (!have[j]) have[j] = slot_take(slots + es[j], buf[j]);
-            missing = missing || !have[j];
-        }
-        if (!__any(missing)) break;
-        __builtin_amdgcn_s_sleep(1);
-        ++spin;
-        if ((spin & 255) == 0 && __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            return false;
-        if (spin > a.spin_limit) {
-            __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-    }
-    double prev = 0.0, qv = 0.0;
-    for (int l = 0; l < WAVE; ++l) {
-        if (lane == l) {
-            double acc1 = acc0, acc2 = 0.0;
-#pragma unroll
-            for (int j = 0; j < PF; ++j)
-                if (j < ne) fold_in<FOLD>(acc1, acc2, (en[j] >> 6) == c ? prev : buf[j], ef[j]);
-            qv = compute(0, acc1, acc2);
-            if (pub_cross) slot_put(slots + my_slot, qv);
-        }
-        prev = readlane_f64(qv, l);
-    }
-    return true;
-}
-
-__device__ __forceinline__ double shfl_up1_f64(const double v) {
-    const uint64_t b = wfh_bits(v);
-    const uint32_t lo = (uint32_t)__shfl_up((int)(uint32_t)b, 1u), hi = (uint32_t)__shfl_up((int)(uint32_t)(b >> 32), 1u);
-    return wfh_from_bits(((uint64_t)hi << 32) | lo);
-}
-
-// A family of S <= 4 sub-steps over a chain chunk (as run_chain) as a diagonal wavefront: in
-// round r lane l computes sub-step r - l, with lane l-1's outflow of the same sub-step (computed
-// in round r-1) shifted over from the neighbouring lane, and the inflow from other chunks of all
-// S sub-steps taken beforehand. Each lane computes its sub-steps in order, and its neighbour has
-// read an outflow before it is replaced, so the results are run_family's.
-template <int FOLD, class Compute>
-__device__ __forceinline__ bool run_chain_diag(const RouteArgs& a, const int lane, const int c, const int S,
-                                               const int* __restrict__ up_node, const int* __restrict__ up_slot,
-                                               const double* __restrict__ up_f, const int e0, const int e1,
-                                               uint64_t* slots, const size_t stride, const int my_slot,
-                                               const bool pub_cross, Compute& compute) {
-    constexpr int PF = 4, SM = 4;
-    const int ne = e1 - e0;
-    int en[PF], es[PF];
-    double ef[PF], buf[PF][SM];
-    bool have[PF][SM];
-#pragma unroll
-    for (int j = 0; j < PF; ++j) {
-        const bool use = j < ne;
-        const int ej = use ? e0 + j : (ne > 0 ? e0 : 0);
-        en[j] = use ? up_node[ej] : c * WAVE;
-        es[j] = use ? up_slot[ej] : 0;
-        ef[j] = (use && FOLD != FOLD_RIV && FOLD != FOLD_SNOW) ? up_f[ej] : 0.0;
-#pragma unroll
-        for (int k = 0; k < SM; ++k) {
-            buf[j][k] = 0.0;
-            have[j][k] = !use || (en[j] >> 6) == c || k >= S;
-        }
-    }
-    long spin = 0;
-    for (;;) {
-        bool missing = false;
-#pragma unroll
-        for (int j = 0; j < PF; ++j)
-#pragma unroll
-            for (int k = 0; k < SM; ++k) {
-                if (!have[j][k]) have[j][k] = slot_take(slots + (size_t)k * stride + es[j], buf[j][k]);
-                missing = missing || !have[j][k];
-            }
-        if (!__any(missing)) break;
-        __builtin_amdgcn_s_sleep(1);
-        ++spin;
-        if ((spin & 255) == 0 && __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            return false;
-        if (spin > a.spin_limit) {
-            __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-    }
-    double qv = 0.0;
-    for (int r = 0; r < WAVE + S - 1; ++r) {
-        const double from_prev = shfl_up1_f64(qv);
-        const int k = r - lane;
-        if (k >= 0 && k < S) {
-            double acc1 = 0.0, acc2 = 0.0;
-#pragma unroll
-            for (int j = 0; j < PF; ++j) {
-                double bk = buf[j][0];
-#pragma unroll
-                for (int kk = 1; kk < SM; ++kk) bk = k == kk ? buf[j][kk] : bk;
-                if (j < ne) fold_in<FOLD>(acc1, acc2, (en[j] >> 6) == c ? from_prev : bk, ef[j]);
-            }
-            qv = compute(k, acc1, acc2);
-            if (pub_cross) slot_put(slots + (size_t)k * stride + my_slot, qv);
-        }
-    }
     return true;
 }
 
@@ -974,6 +917,112 @@ struct SsfEnd {
     double usd, swd, s_tor_avg, o_inwater;
 };
 
+// One lane's subsurface sub-steps. solve() holds what the next cell downstream waits for, account()
+// the sums it does not.
+template <int N>
+struct SsfLane {
+    Column<N> col;
+    double sq, szi;  // discharge and water table depth
+    SsfCum cum{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double area, dsoil, sy, slope, flen, fw, qmax, kh0, fk, zexp, flux;
+    double flx, qin, tor, exf, net;  // of the last sub-step
+    SsfPrep pp;
+    SsfQuick quick;
+    bool col_upd = false;  // the column's closing update is still to be applied
+    double col_z0 = 0.0, col_z1 = 0.0;
+
+    __device__ __forceinline__ void set(const double recharge, const double area_, const double dsoil_, const double sy_,
+                                        const double slope_, const double flen_, const double fw_, const double qmax_,
+                                        const double kh0_, const double fk_, const double zexp_) {
+        area = area_, dsoil = dsoil_, sy = sy_, slope = slope_, flen = flen_, fw = fw_, qmax = qmax_, kh0 = kh0_;
+        fk = fk_, zexp = zexp_;
+        flux = recharge * area;
+    }
+    // everything of the next sub-step that does not depend on its inflow (quick: the column's
+    // update can wait until finish(), that is, the sub-step is the step's last)
+    __device__ __forceinline__ void prepare(const double dts, const bool last) {
+        // flux!(::RechargeModel) with check_flux  boundary_conditions.jl:12-21,219-236
+        flx = szi >= dsoil ? wfh_max(0.0, flux) : flux;
+        pp = ssf_prepare(sq, szi, slope, sy, dts, flen, kh0, fk, zexp);
+        quick = ssf_quick_prepare<N>(sq, szi, 0.0 + flx, sy, dsoil, dts, flen, fw, qmax, pp, col);
+        quick.ok = quick.ok && last;
+    }
+    // The solve's straight part; `open` when it is one for complete().
+    __device__ __forceinline__ double solve(const double dts, const double qin_, const double tor_, bool& open) {
+        qin = qin_, tor = tor_;
+        double qn, zin;
+        bool deferred;
+        open = !ssf_quick_solve(qin, sq, szi, 0.0 + flx, sy, dsoil, dts, pp, quick, qn, zin, exf, net, deferred);
+        if (!open) take(qn, zin, deferred);
+        return qn;
+    }
+    // last: the step's last sub-step, whose column update is left to finish() (nothing reads the
+    // column before that)
+    __device__ __forceinline__ double complete(const double dts, const bool last) {
+        double qn, zin;
+        const bool deferred = kinematic_wave_ssf<N>(qin, sq, szi, 0.0 + flx, slope, sy, dsoil, dts, flen, fw, qmax, kh0,
+                                                    fk, zexp, pp, col, last, qn, zin, exf, net);
+        take(qn, zin, deferred);
+        return qn;
+    }
+    __device__ __forceinline__ void take(const double qn, const double zin, const bool deferred) {
+        col_upd = deferred;
+        col_z0 = szi;
+        col_z1 = zin;
+        sq = qn;
+        szi = zin;
+    }
+    __device__ __forceinline__ void account(const double dts) {
+        cum.rech += flx * dts;
+        cum.tor += tor * dts;
+        cum.qin += qin * dts;
+        cum.q += sq * dts;
+        cum.exf += exf * dts;
+        cum.qnet += net * area * dts;
+    }
+    __device__ __forceinline__ void finish() {
+        if (col_upd) update_ustorelayerdepth<N>(col, col_z0, col_z1);
+    }
+};
+
+// One lane's kinematic-wave sub-steps (overland: DRY, or river), split in the same way.
+template <bool DRY>
+struct KwLane {
+    double q, qin = 0.0, area = 0.0;  // discharge, inflow and flow area of the last sub-step
+    double q_cum = 0.0, qin_cum = 0.0;
+    double q_lat, alpha;
+    bool range_ok;
+    KwPrep p;
+    KwRun run;
+
+    // dt_dx0, dt_dx1: the values of dt / dx that prepare() will get
+    __device__ __forceinline__ void init(const double q0, const double lateral, const double alpha_, const double dt_dx0,
+                                         const double dt_dx1) {
+        q = q0, q_lat = lateral, alpha = alpha_;
+        range_ok = kw_range_ok(dt_dx0, alpha) && kw_range_ok(dt_dx1, alpha);
+    }
+    __device__ __forceinline__ void prepare(const double dts, const double dt_dx) {
+        p = kw_prepare_dx(q, q_lat, alpha, dts, dt_dx, range_ok);
+    }
+    __device__ __forceinline__ double solve(const double inflow, bool& open) {
+        qin = inflow;
+        run = kw_begin<DRY>(qin, p, alpha);
+        open = run.live || run.any;
+        kw_result(run, alpha, q, area);
+        return q;
+    }
+    __device__ __forceinline__ double complete() {
+        kw_end(qin, p, alpha, run);
+        kw_result(run, alpha, q, area);
+        return q;
+    }
+    __device__ __forceinline__ void account(const double dts) {
+        q_cum += q * dts;
+        qin_cum += qin * dts;
+    }
+};
+
+
 // average_flux_vars! (groundwater.jl:630-636), update_soil_water_storage! (soil.jl:1294-1392),
 // the subsurface and land balances (mass_balance.jl:215-253, 470-490) and the overland lateral
 // inflow (surface_kinwave.jl:740-766) of cell p after its last subsurface sub-step.
@@ -1145,12 +1194,12 @@ template <int N, bool EXT, bool MULTI = false, bool FUSE = false>
 __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_eu(route_waves(N)))) k_route(
     const Dev d_arg, const RouteArgs a_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
-    __shared__ int x_k[ROUTE_BLOCK];     // per-wave exchange tables of the routing families
-    __shared__ double x_q[ROUTE_BLOCK];
-    // the wave's table base, wave-uniform (a scalar register rather than a vector one per lane)
-    const int wbase = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~(WAVE - 1)));
-    int* const lds_k = x_k + wbase;
-    double* const lds_q = x_q + wbase;
+    // per-wave table and inbox of the routing families (run_sched); the wave's base is wave-uniform
+    // (a scalar register rather than a vector one per lane)
+    __shared__ double x_q[ROUTE_BLOCK / WAVE * SCHED_RING * SCHED_ROWS];
+    double* const lds_q =
+        x_q + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) * (SCHED_RING * SCHED_ROWS);
+    sched_init<SCHED_RING>(lds_q, lane);
     if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;  // next launch's counter
     for (;;) {
         const RouteKernelArgs& args = kernel_args<RouteKernelArgs>();
@@ -1160,9 +1209,7 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
         const double dt = d.dt;
         const unsigned long long tickets =
             (unsigned long long)a.nchunks * (MULTI ? (unsigned long long)a.nsteps : 1ull);
-        unsigned long long t = 0;
-        if (lane == 0) t = atomicAdd(&a.counters[a.parity], 1ull);
-        t = __shfl(t, 0);
+        const unsigned long long t = next_ticket(&a.counters[a.parity], lane);
         if (t >= tickets) break;
         const int c = MULTI ? (int)(t % (unsigned long long)a.nchunks) : (int)t;
         const int step = MULTI ? (int)(t / (unsigned long long)a.nchunks) : 0;
@@ -1225,47 +1272,30 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
         col.n_unsat = set_layerthickness<N>(col.zi, col.cum, col.act, col.thick);
         col.theta_e = ts - tr;
         col.theta_fc_r = tfc - tr;
-        double sq = ldv<MULTI>(d.ssf_q + q_), szi = col.zi;  // sbm_model.jl:80 hands the soil water table over
-        SsfCum cum{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        // Inflow-independent part of the first sub-step's solve, evaluated before the chain
-        // reaches this cell; the closing soil-column update of the last sub-step is applied
-        // after the family (nothing in the family reads the column after that solve).
-        SsfPrep pp = ssf_prepare(sq, szi, slope, sy, a.S_s == 1 ? a.dts_s[1] : a.dts_s[0], flen, kh0, fk, zexp);
-        bool col_upd = false;
-        double col_z0 = 0.0, col_z1 = 0.0;
-        auto ssf_compute = [&](int k, double qin, double tor) -> double {
-            const double dts = (k == a.S_s - 1) ? a.dts_s[1] : a.dts_s[0];
-            if (k > 0) pp = ssf_prepare(sq, szi, slope, sy, dts, flen, kh0, fk, zexp);
-            // flux!(::RechargeModel) with check_flux  boundary_conditions.jl:12-21,219-236
-            double flx = rech * area;
-            if (szi >= dsoil) flx = wfh_max(0.0, flx);
-            cum.rech += flx * dts;
-            const double qnb = 0.0 + flx;
-            cum.tor += tor * dts;
-            double qn, zin, exf, net;
-            if (kinematic_wave_ssf<N>(qin, sq, szi, qnb, slope, sy, dsoil, dts, flen, fw, qmax, kh0, fk, zexp, pp,
-                                      col, k == a.S_s - 1, qn, zin, exf, net)) {
-                col_upd = true;
-                col_z0 = szi;
-                col_z1 = zin;
-            }
-            sq = qn;
-            szi = zin;
-            cum.qin += qin * dts;
-            cum.q += qn * dts;
-            cum.exf += exf * dts;
-            cum.qnet += net * area * dts;
-            return qn;
+        SsfLane<N> ssf;
+        ssf.col = col;
+        ssf.sq = ldv<MULTI>(d.ssf_q + q_);
+        ssf.szi = col.zi;  // sbm_model.jl:80 hands the soil water table over
+        ssf.set(rech, area, dsoil, sy, slope, flen, fw, qmax, kh0, fk, zexp);
+        ssf.prepare(a.S_s == 1 ? a.dts_s[1] : a.dts_s[0], a.S_s == 1);
+        const auto ssf_compute = [&](const int k, const double qin, const double tor, bool& open) ROUTE_INLINE -> double {
+            return ssf.solve(k == a.S_s - 1 ? a.dts_s[1] : a.dts_s[0], qin, tor, open);
         };
-        const bool lchain = d.chain_land[c] != 0;  // wave-uniform
-        if (lchain && a.S_s == 1
-                ? !run_chain<FOLD_SSF>(a, lane, c, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ssf, p,
-                                       (fl & 1) && !lcons_in, ssf_compute)
-                : !run_family<FOLD_SSF>(a, lane, c, valid, a.S_s, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ssf,
-                                        (size_t)n, p, (fl & 1) && !lcons_in, lcons_in ? (dn & 63) : -1, lds_k, lds_q,
-                                        ssf_compute))
+        const auto ssf_complete = [&](const int k) ROUTE_INLINE -> double {
+            return ssf.complete(k == a.S_s - 1 ? a.dts_s[1] : a.dts_s[0], k == a.S_s - 1);
+        };
+        const auto ssf_after = [&](const int k) ROUTE_INLINE {
+            ssf.account(k == a.S_s - 1 ? a.dts_s[1] : a.dts_s[0]);
+            if (k < a.S_s - 1) ssf.prepare(k + 1 == a.S_s - 1 ? a.dts_s[1] : a.dts_s[0], k + 1 == a.S_s - 1);
+        };
+        const int lrank = d.rank_land[q_], lnrank = __builtin_amdgcn_readfirstlane(d.nrank_land[c]);
+        if (!run_sched<FOLD_SSF, SCHED_RING>(a, lane, c, valid, a.S_s, lrank, lnrank, d.up_idx, d.up_idx, d.up_f, e0, e1,
+                                             a.slot_ssf, (size_t)n, p, (fl & 1) && !lcons_in, lds_q, ssf_compute,
+                                             ssf_complete, ssf_after))
             return;
-        if (col_upd) update_ustorelayerdepth<N>(col, col_z0, col_z1);
+        ssf.finish();
+        const double sq = ssf.sq, szi = ssf.szi;
+        const SsfCum& cum = ssf.cum;
 
         // Inputs of the later phases (soil storage, balances, overland flow), loaded once the
         // subsurface family is done, so that they take no registers while it runs (with FUSE,
@@ -1301,40 +1331,37 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
         // ---------------- average_flux_vars!, update_soil_water_storage! ----------------
         SsfEnd se{0.0, 0.0, 0.0, 0.0};
         if (valid)
-            se = ssf_finish<N, MULTI>(d, p, col,
+            se = ssf_finish<N, MULTI>(d, p, ssf.col,
                                SsfCellIn{ts, tr, rd, dsoil, area, sy, sat_exc, runoff_l, inf_exc, aeow, nrr, P_in, aet,
                                          leak, canopy, snow_s, snow_w, store_prev, snow_in, snow_out},
                                cum, sq, szi);
         const double o_inwater = se.o_inwater, s_tor_avg = se.s_tor_avg, usd = se.usd, swd = se.swd;
 
         // ---------------- overland kinematic wave ----------------
-        const double oqlat = o_inwater / flen;
-        double oq = oq0, oh = oh0, o_storage = 0.0, oqin = 0.0;
-        double o_q_cum = 0.0, o_qin_cum = 0.0, o_tor_cum = 0.0;
-        KwPrep op = kw_prepare(oq, oqlat, alpha, a.S_l == 1 ? a.dts_l[1] : a.dts_l[0], flen);
-        auto ol_compute = [&](int k, double tor, double qin_all) -> double {
-            const double dts = (k == a.S_l - 1) ? a.dts_l[1] : a.dts_l[0];
-            if (k > 0) op = kw_prepare(oq, oqlat, alpha, dts, flen);
-            o_tor_cum += tor * dts;
-            double qin = 0.0;
-            if (sfw > 0.0) qin = qin_all;
-            double qn, ar;
-            kw_solve(qin, op, alpha, qn, ar);
-            oq = qn;
-            if (sfw > 0.0) oh = ar / sfw;
-            o_storage = flen * sfw * oh;
-            o_q_cum += qn * dts;
-            o_qin_cum += qin * dts;
-            oqin = qin;
-            return qn;
+        KwLane<true> ol;
+        const double o_dx1 = a.dts_l[1] / flen, o_dx0 = a.S_l == 1 ? o_dx1 : a.dts_l[0] / flen;
+        ol.init(oq0, o_inwater / flen, alpha, o_dx0, o_dx1);
+        ol.prepare(a.S_l == 1 ? a.dts_l[1] : a.dts_l[0], o_dx0);
+        double o_tor = 0.0, o_tor_cum = 0.0;
+        const auto ol_compute = [&](int, const double tor, const double qin_all, bool& open) ROUTE_INLINE -> double {
+            o_tor = tor;
+            return ol.solve(sfw > 0.0 ? qin_all : 0.0, open);
         };
-        if (lchain && a.S_l == 1
-                ? !run_chain<FOLD_OL>(a, lane, c, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ol, p,
-                                      (fl & 1) && !lcons_in, ol_compute)
-                : !run_family<FOLD_OL>(a, lane, c, valid, a.S_l, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ol,
-                                       (size_t)n, p, (fl & 1) && !lcons_in, lcons_in ? (dn & 63) : -1, lds_k, lds_q,
-                                       ol_compute))
+        const auto ol_complete = [&](int) ROUTE_INLINE -> double { return ol.complete(); };
+        const auto ol_after = [&](const int k) ROUTE_INLINE {
+            const double dts = k == a.S_l - 1 ? a.dts_l[1] : a.dts_l[0];
+            o_tor_cum += o_tor * dts;
+            ol.account(dts);
+            if (k < a.S_l - 1)
+                ol.prepare(k + 1 == a.S_l - 1 ? a.dts_l[1] : a.dts_l[0], k + 1 == a.S_l - 1 ? o_dx1 : o_dx0);
+        };
+        if (!run_sched<FOLD_OL, SCHED_RING>(a, lane, c, valid, a.S_l, lrank, lnrank, d.up_idx, d.up_idx, d.up_f, e0, e1,
+                                            a.slot_ol, (size_t)n, p, (fl & 1) && !lcons_in, lds_q, ol_compute,
+                                            ol_complete, ol_after))
             return;
+        // the last sub-step's depth and storage
+        const double oh = sfw > 0.0 ? ol.area / sfw : oh0;
+        const double o_storage = flen * sfw * oh;
         // inputs of the river phase, loaded once the overland family is done
         const int r_ = d.river_of[q_];
         const int r = valid ? r_ : -1;
@@ -1348,44 +1375,47 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
                      r_store_prev = ldv<MULTI>(d.r_storage + rr);
         double r_inwater = 0.0;
         if (valid)
-            r_inwater = ol_finish<MULTI>(d, p, r, oq, oh, o_storage, oqin, o_q_cum, o_tor_cum, o_qin_cum, o_inwater,
+            r_inwater = ol_finish<MULTI>(d, p, r, ol.q, oh, o_storage, ol.qin, ol.q_cum, o_tor_cum, ol.qin_cum, o_inwater,
                                          o_store_prev, s_tor_avg, nrr, area, rarea);
 
         // ---------------- river kinematic wave ----------------
         const bool rcons_in = riv && (fl & 4) && cons_in;  // a river cell drains to the land downstream
         const double rqlat = r_inwater / rfl;
-        double rq = rq0, rh = rh0, r_storage = 0.0, rqin = 0.0;
-        double r_q_cum = 0.0, r_qin_cum = 0.0;
         double inflow = 0.0 / rfl;  // reservoir / lake / external inflow terms (none in this model)
         inflow -= 0.0 / rfl;
-        const double rqlat_all = rqlat + inflow;
-        KwPrep rp = kw_prepare(rq, rqlat_all, ralpha, a.S_r == 1 ? a.dts_r[1] : a.dts_r[0], rfl);
-        auto riv_compute = [&](int k, double sumq, double res_out) -> double {
-            const double dts = (k == a.S_r - 1) ? a.dts_r[1] : a.dts_r[0];
-            if (k > 0) rp = kw_prepare(rq, rqlat_all, ralpha, dts, rfl);
-            const double qin = (EXT ? res_out : 0.0) + sumq;
-            double qn, ar;
-            kw_solve(qin, rp, ralpha, qn, ar);
-            rq = qn;
-            rh = ar / rfw;
-            r_storage = rfl * ar;
-            r_q_cum += qn * dts;
-            r_qin_cum += qin * dts;
-            rqin = qin;
-            if (EXT && rres >= 0) return reservoir_step(d, rres, p, qn, dts, k == 0, k == a.S_r - 1);
+        KwLane<false> rv;
+        const double r_dx1 = a.dts_r[1] / rfl, r_dx0 = a.S_r == 1 ? r_dx1 : a.dts_r[0] / rfl;
+        rv.init(rq0, rqlat + inflow, ralpha, r_dx0, r_dx1);
+        rv.prepare(a.S_r == 1 ? a.dts_r[1] : a.dts_r[0], r_dx0);
+        // what the cell passes on: its discharge, or its reservoir's outflow
+        const auto riv_out = [&](const int k, const double qn) ROUTE_INLINE -> double {
+            if (EXT && rres >= 0)
+                return reservoir_step(d, rres, p, qn, k == a.S_r - 1 ? a.dts_r[1] : a.dts_r[0], k == 0, k == a.S_r - 1);
             return qn;
         };
-        if (d.chain_rl[c] != 0 && a.S_r <= 4
-                ? !run_chain_diag<EXT ? FOLD_RIV_RES : FOLD_RIV>(a, lane, c, a.S_r, d.rup_node, d.rup_idx, d.rup_res,
-                                                                 re0, re1, a.slot_r, (size_t)d.nriv, rr,
-                                                                 riv && (fl & 4) && !rcons_in, riv_compute)
-                : !run_family<EXT ? FOLD_RIV_RES : FOLD_RIV>(a, lane, c, riv, a.S_r, d.rup_node, d.rup_idx,
-                                                             d.rup_res, re0, re1, a.slot_r, (size_t)d.nriv, rr,
-                                                             riv && (fl & 4) && !rcons_in,
-                                                             rcons_in ? (dn & 63) : -1, lds_k, lds_q, riv_compute))
+        const auto riv_compute = [&](const int k, const double sumq, const double res_out,
+                                     bool& open) ROUTE_INLINE -> double {
+            const double qn = rv.solve((EXT ? res_out : 0.0) + sumq, open);
+            if (EXT) open = open || rres >= 0;
+            return qn;
+        };
+        const auto riv_complete = [&](const int k) ROUTE_INLINE -> double { return riv_out(k, rv.complete()); };
+        const auto riv_after = [&](const int k) ROUTE_INLINE {
+            rv.account(k == a.S_r - 1 ? a.dts_r[1] : a.dts_r[0]);
+            if (k < a.S_r - 1)
+                rv.prepare(k + 1 == a.S_r - 1 ? a.dts_r[1] : a.dts_r[0], k + 1 == a.S_r - 1 ? r_dx1 : r_dx0);
+        };
+        if (!run_sched<EXT ? FOLD_RIV_RES : FOLD_RIV, SCHED_RING>(
+                a, lane, c, riv, a.S_r, d.rank_riv[q_],
+                __builtin_amdgcn_readfirstlane(d.nrank_riv[c]), d.rup_node, d.rup_idx, d.rup_res, re0, re1,
+                a.slot_r, (size_t)d.nriv, rr, riv && (fl & 4) && !rcons_in, lds_q, riv_compute, riv_complete,
+                riv_after))
             return;
-        if (riv) riv_finish<MULTI>(d, r, rq, rh, r_storage, rqin, r_q_cum, r_qin_cum, r_inwater, r_store_prev);
-        if (MULTI && riv && a.run_q_avg) a.run_q_avg[(size_t)step * d.nriv + r] = r_q_cum / dt;
+        // the last sub-step's depth and storage
+        const double rh = riv ? rv.area / rfw : rh0;
+        const double r_storage = rfl * rv.area;
+        if (riv) riv_finish<MULTI>(d, r, rv.q, rh, r_storage, rv.qin, rv.q_cum, rv.qin_cum, r_inwater, r_store_prev);
+        if (MULTI && riv && a.run_q_avg) a.run_q_avg[(size_t)step * d.nriv + r] = rv.q_cum / dt;
 
         // ---------------- update_total_water_storage!  sbm.jl:143-182 ----------------
         if (valid)
@@ -1409,9 +1439,7 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
 // update_river_flow_model! :613-662).
 // ============================================================================================
 #define AD_TICKET(NCHUNKS)                                                       \
-    unsigned long long t_ = 0;                                                   \
-    if (lane == 0) t_ = atomicAdd(&a.counters[a.parity], 1ull);                  \
-    t_ = __shfl(t_, 0);                                                          \
+    const unsigned long long t_ = next_ticket(&a.counters[a.parity], lane);      \
     if (t_ >= (unsigned long long)(NCHUNKS)) break;                              \
     const int c = (int)t_;
 
@@ -1421,10 +1449,9 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ssf(const Dev d_arg, const R
                                                         const AdArgs x_arg, const double dts_arg, const int first_arg,
                                                         const int last_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
-    __shared__ int x_k[ROUTE_BLOCK];
-    __shared__ double x_q[ROUTE_BLOCK];
-    int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
-    double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
+    __shared__ double x_q[ROUTE_BLOCK / WAVE * SCHED_ROWS];
+    double* const lds_q = x_q + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) * SCHED_ROWS;
+    sched_init<1>(lds_q, lane);
     if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
         const AdKernelArgs& args = kernel_args<AdKernelArgs>();
@@ -1457,56 +1484,39 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ssf(const Dev d_arg, const R
         col.n_unsat = set_layerthickness<N>(col.zi, col.cum, col.act, col.thick);
         col.theta_e = ts - tr;
         col.theta_fc_r = tfc - tr;
-        double sq = d.ssf_q[q_], szi = x.szi[q_];
-        SsfCum cum{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        SsfLane<N> ssf;
+        ssf.col = col;
+        ssf.sq = d.ssf_q[q_];
+        ssf.szi = x.szi[q_];
+        ssf.set(rech, area, dsoil, sy, slope, flen, fw, qmax, kh0, fk, zexp);
         if (!first) {
-            cum.qin = x.scum[q_];
-            cum.q = x.scum[(size_t)n + q_];
-            cum.exf = x.scum[2 * (size_t)n + q_];
-            cum.qnet = x.scum[3 * (size_t)n + q_];
-            cum.tor = x.scum[4 * (size_t)n + q_];
-            cum.rech = x.scum[5 * (size_t)n + q_];
+            ssf.cum.qin = x.scum[q_];
+            ssf.cum.q = x.scum[(size_t)n + q_];
+            ssf.cum.exf = x.scum[2 * (size_t)n + q_];
+            ssf.cum.qnet = x.scum[3 * (size_t)n + q_];
+            ssf.cum.tor = x.scum[4 * (size_t)n + q_];
+            ssf.cum.rech = x.scum[5 * (size_t)n + q_];
         }
-        const SsfPrep pp = ssf_prepare(sq, szi, slope, sy, dts, flen, kh0, fk, zexp);
-        bool col_upd = false;
-        double col_z0 = 0.0, col_z1 = 0.0;
-        auto ssf_compute = [&](int, double qin, double tor) -> double {
-            // flux!(::RechargeModel) with check_flux  boundary_conditions.jl:12-21,219-236
-            double flx = rech * area;
-            if (szi >= dsoil) flx = wfh_max(0.0, flx);
-            cum.rech += flx * dts;
-            const double qnb = 0.0 + flx;
-            cum.tor += tor * dts;
-            double qn, zin, exf, net;
-            if (kinematic_wave_ssf<N>(qin, sq, szi, qnb, slope, sy, dsoil, dts, flen, fw, qmax, kh0, fk, zexp, pp, col,
-                                      true,
-                                      qn, zin, exf, net)) {
-                col_upd = true;
-                col_z0 = szi;
-                col_z1 = zin;
-            }
-            sq = qn;
-            szi = zin;
-            cum.qin += qin * dts;
-            cum.q += qn * dts;
-            cum.exf += exf * dts;
-            cum.qnet += net * area * dts;
-            return qn;
+        ssf.prepare(dts, true);
+        const auto ssf_compute = [&](int, const double qin, const double tor, bool& open) ROUTE_INLINE -> double {
+            return ssf.solve(dts, qin, tor, open);
         };
-        if (d.chain_land[c] != 0
-                ? !run_chain<FOLD_SSF>(a, lane, c, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ssf, p,
-                                       (fl & 1) && !cons_in, ssf_compute)
-                : !run_family<FOLD_SSF>(a, lane, c, valid, 1, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ssf,
-                                        (size_t)n, p, (fl & 1) && !cons_in, cons_in ? (dn & 63) : -1, lds_k, lds_q,
-                                        ssf_compute))
+        const auto ssf_complete = [&](int) ROUTE_INLINE -> double { return ssf.complete(dts, true); };
+        const auto ssf_after = [&](int) ROUTE_INLINE { ssf.account(dts); };
+        if (!run_sched<FOLD_SSF, 1>(a, lane, c, valid, 1, d.rank_land[q_],
+                                    __builtin_amdgcn_readfirstlane(d.nrank_land[c]), d.up_idx, d.up_idx, d.up_f, e0,
+                                    e1, a.slot_ssf, (size_t)n, p, (fl & 1) && !cons_in, lds_q, ssf_compute,
+                                    ssf_complete, ssf_after))
             return;
-        if (col_upd) update_ustorelayerdepth<N>(col, col_z0, col_z1);
+        ssf.finish();
+        const double sq = ssf.sq, szi = ssf.szi;
+        const SsfCum& cum = ssf.cum;
         if (valid && !last) {
             d.ssf_q[p] = sq;
             x.szi[p] = szi;
-            d.zi[p] = col.zi;
+            d.zi[p] = ssf.col.zi;
 #pragma unroll
-            for (int k = 0; k < N; ++k) d.ustore[k * n + p] = col.ustore[k];
+            for (int k = 0; k < N; ++k) d.ustore[k * n + p] = ssf.col.ustore[k];
             x.scum[p] = cum.qin;
             x.scum[(size_t)n + p] = cum.q;
             x.scum[2 * (size_t)n + p] = cum.exf;
@@ -1517,7 +1527,7 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ssf(const Dev d_arg, const R
             const double P_in = d.balance && !(d.flags[p] & 8) ? d.P[p] : 0.0, aet = d.balance ? d.aet[p] : 0.0;
             const double leak = d.balance ? d.leakage[p] : 0.0, sp = d.balance ? d.store_prev[p] : 0.0;
             const double ss = d.snow ? d.snow_s[p] : 0.0, sw = d.snow ? d.snow_w[p] : 0.0;
-            ssf_finish<N>(d, p, col,
+            ssf_finish<N>(d, p, ssf.col,
                           SsfCellIn{ts, tr, ld(d.rd, p), dsoil, area, sy, d.sat_excess[p], d.runoff_land[p],
                                     d.inf_excess[p], d.aeow_l[p], d.net_runoff_river[p], P_in, aet, leak, d.canopy[p],
                                     ss, sw, sp, d.snow_in[p], d.snow_out[p]},
@@ -1531,10 +1541,9 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ol(const Dev d_arg, const Ro
                                                         const AdArgs x_arg, const double dts_arg, const int first_arg,
                                                         const int last_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
-    __shared__ int x_k[ROUTE_BLOCK];
-    __shared__ double x_q[ROUTE_BLOCK];
-    int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
-    double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
+    __shared__ double x_q[ROUTE_BLOCK / WAVE * SCHED_ROWS];
+    double* const lds_q = x_q + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) * SCHED_ROWS;
+    sched_init<1>(lds_q, lane);
     if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
         const AdKernelArgs& args = kernel_args<AdKernelArgs>();
@@ -1555,48 +1564,44 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_ol(const Dev d_arg, const Ro
         const bool cons_in = dn >= 0 && (dn >> 6) == c && (fl & 1);  // a reservoir outlet feeds no land cell
         const int e1 = valid ? e1_ : e0;
         const double alpha = ld(d.alpha, q_), sfw = ld(d.sfw, q_), flen = ld(d.fl, q_);
-        double oq = d.ol_q[q_], oh = d.ol_h[q_];
+        const double oh0 = d.ol_h[q_];
         const double o_inwater = d.ol_inwater[q_];
-        double o_q_cum = 0.0, o_qin_cum = 0.0, o_tor_cum = 0.0;
+        KwLane<true> ol;
+        const double o_dx = dts / flen;
+        ol.init(d.ol_q[q_], o_inwater / flen, alpha, o_dx, o_dx);
+        double o_tor = 0.0, o_tor_cum = 0.0;
         if (!first) {
-            o_q_cum = x.ocum[q_];
-            o_qin_cum = x.ocum[(size_t)n + q_];
+            ol.q_cum = x.ocum[q_];
+            ol.qin_cum = x.ocum[(size_t)n + q_];
             o_tor_cum = x.ocum[2 * (size_t)n + q_];
         }
-        const double oqlat = o_inwater / flen;
-        double o_storage = 0.0, oqin = 0.0;
-        const KwPrep op = kw_prepare(oq, oqlat, alpha, dts, flen);
-        auto ol_compute = [&](int, double tor, double qin_all) -> double {
-            o_tor_cum += tor * dts;
-            double qin = 0.0;
-            if (sfw > 0.0) qin = qin_all;
-            double qn, ar;
-            kw_solve(qin, op, alpha, qn, ar);
-            oq = qn;
-            if (sfw > 0.0) oh = ar / sfw;
-            o_storage = flen * sfw * oh;
-            o_q_cum += qn * dts;
-            o_qin_cum += qin * dts;
-            oqin = qin;
-            return qn;
+        ol.prepare(dts, o_dx);
+        const auto ol_compute = [&](int, const double tor, const double qin_all, bool& open) ROUTE_INLINE -> double {
+            o_tor = tor;
+            return ol.solve(sfw > 0.0 ? qin_all : 0.0, open);
         };
-        if (d.chain_land[c] != 0
-                ? !run_chain<FOLD_OL>(a, lane, c, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ol, p,
-                                      (fl & 1) && !cons_in, ol_compute)
-                : !run_family<FOLD_OL>(a, lane, c, valid, 1, d.up_idx, d.up_idx, d.up_f, e0, e1, a.slot_ol,
-                                       (size_t)n, p, (fl & 1) && !cons_in, cons_in ? (dn & 63) : -1, lds_k, lds_q,
-                                       ol_compute))
+        const auto ol_complete = [&](int) ROUTE_INLINE -> double { return ol.complete(); };
+        const auto ol_after = [&](int) ROUTE_INLINE {
+            o_tor_cum += o_tor * dts;
+            ol.account(dts);
+        };
+        if (!run_sched<FOLD_OL, 1>(a, lane, c, valid, 1, d.rank_land[q_],
+                                    __builtin_amdgcn_readfirstlane(d.nrank_land[c]), d.up_idx, d.up_idx, d.up_f, e0,
+                                   e1, a.slot_ol, (size_t)n, p, (fl & 1) && !cons_in, lds_q, ol_compute,
+                                   ol_complete, ol_after))
             return;
+        const double oh = sfw > 0.0 ? ol.area / sfw : oh0;
+        const double o_storage = flen * sfw * oh;
         if (valid && !last) {
-            d.ol_q[p] = oq;
+            d.ol_q[p] = ol.q;
             d.ol_h[p] = oh;
-            x.ocum[p] = o_q_cum;
-            x.ocum[(size_t)n + p] = o_qin_cum;
+            x.ocum[p] = ol.q_cum;
+            x.ocum[(size_t)n + p] = ol.qin_cum;
             x.ocum[2 * (size_t)n + p] = o_tor_cum;
         } else if (valid) {
             const int r = d.river_of[p];
             const double o_store_prev = d.ol_storage[p];
-            ol_finish(d, p, r, oq, oh, o_storage, oqin, o_q_cum, o_tor_cum, o_qin_cum, o_inwater, o_store_prev,
+            ol_finish(d, p, r, ol.q, oh, o_storage, ol.qin, ol.q_cum, o_tor_cum, ol.qin_cum, o_inwater, o_store_prev,
                       d.ssf_tor_avg[p], d.net_runoff_river[p], ld(d.area, p), r >= 0 ? d.r_area[r] : 0.0);
         }
     }
@@ -1695,10 +1700,9 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_riv(const Dev d_arg, const R
                                                         const AdArgs x_arg, const double dts_arg, const int first_arg,
                                                         const int last_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
-    __shared__ int x_k[ROUTE_BLOCK];
-    __shared__ double x_q[ROUTE_BLOCK];
-    int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
-    double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
+    __shared__ double x_q[ROUTE_BLOCK / WAVE * SCHED_ROWS];
+    double* const lds_q = x_q + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) * SCHED_ROWS;
+    sched_init<1>(lds_q, lane);
     if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
         const AdKernelArgs& args = kernel_args<AdKernelArgs>();
@@ -1718,12 +1722,11 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_riv(const Dev d_arg, const R
         const bool cons_in = rdn >= 0 && (rdn >> 6) == c;
         const int e1 = valid ? e1_ : e0;
         const double ralpha = d.r_alpha[r], rfw = d.r_fw[r], rfl = d.r_fl[r];
-        double rq = d.r_q[r], rh = d.r_h[r];
         const double r_inwater = d.r_inwater[r];
-        double r_q_cum = 0.0, r_qin_cum = 0.0;
+        KwLane<false> rv;
         if (!first) {
-            r_q_cum = x.rcum[q_];
-            r_qin_cum = x.rcum[(size_t)nr + q_];
+            rv.q_cum = x.rcum[q_];
+            rv.qin_cum = x.rcum[(size_t)nr + q_];
         }
         const double rqlat = r_inwater / rfl;
         double fs = 0.0, fh = 0.0, fexch = 0.0;
@@ -1731,50 +1734,46 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_riv(const Dev d_arg, const R
         double inflow = 0.0 / rfl;  // reservoir / lake / external inflow terms (none in this model)
         inflow -= 0.0 / rfl;
         if (FP) inflow += fexch / rfl;  // channel-floodplain exchange (surface_kinwave.jl:534-536)
-        const double rqlat_all = rqlat + inflow;
-        double r_storage = 0.0, rqin = 0.0;
-        const KwPrep rpp = kw_prepare(rq, rqlat_all, ralpha, dts, rfl);
+        const double r_dx = dts / rfl;
+        rv.init(d.r_q[r], rqlat + inflow, ralpha, r_dx, r_dx);
+        rv.prepare(dts, r_dx);
         const int rres_ = RES ? d.res_of_r[r] : -1, pnode = RES ? x.rp_node[q_] : 0;
         const int rres = valid ? rres_ : -1;
-        auto riv_compute = [&](int, double sumq, double res_out) -> double {
-            const double qin = (RES ? res_out : 0.0) + sumq;
-            double qn, ar;
-            kw_solve(qin, rpp, ralpha, qn, ar);
-            rq = qn;
-            rh = ar / rfw;
-            r_storage = rfl * ar;
-            r_q_cum += qn * dts;
-            r_qin_cum += qin * dts;
-            rqin = qin;
+        const auto riv_compute = [&](int, const double sumq, const double res_out, bool& open) ROUTE_INLINE -> double {
+            const double qn = rv.solve((RES ? res_out : 0.0) + sumq, open);
+            if (RES) open = open || rres >= 0;
+            return qn;
+        };
+        const auto riv_complete = [&](int) ROUTE_INLINE -> double {
+            const double qn = rv.complete();
             if (RES && rres >= 0) return reservoir_step<LINK>(d, rres, pnode, qn, dts, first != 0, last != 0);
             return qn;
         };
-        const bool chain = x.chain_r[c] != 0;  // wave-uniform
-        if (chain ? !run_chain<RES ? FOLD_RIV_RES : FOLD_RIV>(a, lane, c, x.rp_up_idx, x.rp_up_idx, x.rp_up_res, e0, e1,
-                                                                a.slot_r, rp, rdn >= 0 && !cons_in, riv_compute)
-                  : !run_family<RES ? FOLD_RIV_RES : FOLD_RIV>(a, lane, c, valid, 1, x.rp_up_idx, x.rp_up_idx,
-                                                                 x.rp_up_res, e0, e1, a.slot_r, (size_t)nr, rp,
-                                                                 rdn >= 0 && !cons_in, cons_in ? (rdn & 63) : -1,
-                                                                 lds_k, lds_q, riv_compute))
+        const auto riv_after = [&](int) ROUTE_INLINE { rv.account(dts); };
+        const int rrank = x.rank_r[q_], rnrank = __builtin_amdgcn_readfirstlane(x.nrank_r[c]);
+        if (!run_sched<RES ? FOLD_RIV_RES : FOLD_RIV, 1>(a, lane, c, valid, 1, rrank, rnrank, x.rp_up_idx, x.rp_up_idx,
+                                                         x.rp_up_res, e0, e1, a.slot_r, (size_t)nr, rp,
+                                                         rdn >= 0 && !cons_in, lds_q, riv_compute, riv_complete,
+                                                         riv_after))
             return;
+        const double rh = rv.area / rfw;
+        const double r_storage = rfl * rv.area;
         if (FP) {
             const double cap = fp_capacity(d, r, rdn_ >= 0 ? x.rp_r[rdn_] : -1, fh);
             double s_new = fs, flux = 0.0;
-            auto pass = [&](int, double material, double) -> double {
+            auto pass = [&](int, double material, double, bool&) ROUTE_INLINE -> double {
                 const double flux_val = wfh_min(material / dts, cap);
                 const double update = flux_val * dts;
                 s_new = material - update;
                 flux = flux_val;
                 return update;
             };
-            // the floodplain lists hold the same upstream cells as the river's (in another order),
-            // so a chain chunk of the river is one of the floodplain too
+            // the floodplain lists hold the same upstream cells as the river's (in another order), so
+            // the river's ranks hold for them too
             const int f0 = x.fp_sup_ptr[q_], f1 = valid ? x.fp_sup_ptr[q_ + 1] : f0;
-            if (chain ? !run_chain<FOLD_SNOW>(a, lane, c, x.fp_sup_idx, x.fp_sup_idx, nullptr, f0, f1, a.slot_ssf, rp,
-                                              rdn >= 0 && !cons_in, pass, fs)
-                      : !run_family<FOLD_SNOW>(a, lane, c, valid, 1, x.fp_sup_idx, x.fp_sup_idx, nullptr, f0, f1,
-                                               a.slot_ssf, (size_t)nr, rp, rdn >= 0 && !cons_in,
-                                               cons_in ? (rdn & 63) : -1, lds_k, lds_q, pass, fs))
+            if (!run_sched<FOLD_SNOW, 1>(a, lane, c, valid, 1, rrank, rnrank, x.fp_sup_idx, x.fp_sup_idx, nullptr, f0, f1,
+                                         a.slot_ssf, (size_t)nr, rp, rdn >= 0 && !cons_in, lds_q, pass, [](int) { return 0.0; },
+                                         [](int) {}, fs))
                 return;
             if (valid) {
                 if (first) {
@@ -1791,12 +1790,12 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_ad_riv(const Dev d_arg, const R
             }
         }
         if (valid && !last) {
-            d.r_q[r] = rq;
+            d.r_q[r] = rv.q;
             d.r_h[r] = rh;
-            x.rcum[rp] = r_q_cum;
-            x.rcum[(size_t)nr + rp] = r_qin_cum;
+            x.rcum[rp] = rv.q_cum;
+            x.rcum[(size_t)nr + rp] = rv.qin_cum;
         } else if (valid) {
-            riv_finish(d, r, rq, rh, r_storage, rqin, r_q_cum, r_qin_cum, r_inwater, d.r_storage[r]);
+            riv_finish(d, r, rv.q, rh, r_storage, rv.qin, rv.q_cum, rv.qin_cum, r_inwater, d.r_storage[r]);
         }
     }
 }
@@ -1865,10 +1864,9 @@ __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long v)
 // the transport (TAN80 = 5.67, snow_storage_max = 10 m).
 __global__ void __launch_bounds__(ROUTE_BLOCK) k_snow_transport(const Dev d_arg, const RouteArgs a_arg) {
     const int lane = threadIdx.x & (WAVE - 1);
-    __shared__ int x_k[ROUTE_BLOCK];
-    __shared__ double x_q[ROUTE_BLOCK];
-    int* const lds_k = x_k + (threadIdx.x & ~(WAVE - 1));
-    double* const lds_q = x_q + (threadIdx.x & ~(WAVE - 1));
+    __shared__ double x_q[ROUTE_BLOCK / WAVE * SCHED_ROWS];
+    double* const lds_q = x_q + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE)) * SCHED_ROWS;
+    sched_init<1>(lds_q, lane);
     if (blockIdx.x == 0 && threadIdx.x == 0) a_arg.counters[a_arg.parity ^ 1] = 0ull;
     for (;;) {
         const RouteKernelArgs& args = kernel_args<RouteKernelArgs>();
@@ -1888,32 +1886,26 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) k_snow_transport(const Dev d_arg,
         const double frac = wfh_min(0.5, slope / 5.67) * wfh_min(1.0, ss / 10.0);
         const double cap_s = frac * ss / dt, cap_w = sw * frac / dt;
         double ss_new = ss, sw_new = sw, flux_s = 0.0, flux_w = 0.0;
-        auto pass_s = [&](int, double material, double) -> double {
+        auto pass_s = [&](int, double material, double, bool&) ROUTE_INLINE -> double {
             const double flux_val = wfh_min(material / dt, cap_s);
             const double update = flux_val * dt;
             ss_new = material - update;
             flux_s = flux_val;
             return update;
         };
-        const bool chain = d.chain_sup[c] != 0;  // wave-uniform
-        if (chain ? !run_chain<FOLD_SNOW>(a, lane, c, d.sup_idx, d.sup_idx, nullptr, e0, e1, a.slot_ssf, p,
-                                          dn >= 0 && !cons_in, pass_s, ss)
-                  : !run_family<FOLD_SNOW>(a, lane, c, valid, 1, d.sup_idx, d.sup_idx, nullptr, e0, e1, a.slot_ssf,
-                                           (size_t)n, p, dn >= 0 && !cons_in, cons_in ? (dn & 63) : -1, lds_k, lds_q,
-                                           pass_s, ss))
+        const int rank = d.rank_land[q_], nrank = __builtin_amdgcn_readfirstlane(d.nrank_land[c]);
+        if (!run_sched<FOLD_SNOW, 1>(a, lane, c, valid, 1, rank, nrank, d.sup_idx, d.sup_idx, nullptr, e0, e1, a.slot_ssf,
+                                     (size_t)n, p, dn >= 0 && !cons_in, lds_q, pass_s, [](int) { return 0.0; }, [](int) {}, ss))
             return;
-        auto pass_w = [&](int, double material, double) -> double {
+        auto pass_w = [&](int, double material, double, bool&) ROUTE_INLINE -> double {
             const double flux_val = wfh_min(material / dt, cap_w);
             const double update = flux_val * dt;
             sw_new = material - update;
             flux_w = flux_val;
             return update;
         };
-        if (chain ? !run_chain<FOLD_SNOW>(a, lane, c, d.sup_idx, d.sup_idx, nullptr, e0, e1, a.slot_ol, p,
-                                          dn >= 0 && !cons_in, pass_w, sw)
-                  : !run_family<FOLD_SNOW>(a, lane, c, valid, 1, d.sup_idx, d.sup_idx, nullptr, e0, e1, a.slot_ol,
-                                           (size_t)n, p, dn >= 0 && !cons_in, cons_in ? (dn & 63) : -1, lds_k, lds_q,
-                                           pass_w, sw))
+        if (!run_sched<FOLD_SNOW, 1>(a, lane, c, valid, 1, rank, nrank, d.sup_idx, d.sup_idx, nullptr, e0, e1, a.slot_ol,
+                                     (size_t)n, p, dn >= 0 && !cons_in, lds_q, pass_w, [](int) { return 0.0; }, [](int) {}, sw))
             return;
         if (valid) {
             d.snow_s[p] = ss_new;
@@ -2387,6 +2379,39 @@ static double interp_host(double x, const double* xp, const double* fp, int64_t 
     if (i1 < 0 || i1 + 1 >= n) return std::nan("");
     const int64_t i2 = i1 + 1;
     return fp[i1 * fs] * (1.0 - (x - xp[i1]) / (xp[i2] - xp[i1])) + fp[i2 * fs] * (x - xp[i1]) / (xp[i2] - xp[i1]);
+}
+
+// The pass schedule of every chunk of 64 positions (run_sched). A cell of the chunk that drains
+// inside it gets the rank just below its consumer's, so its outflow is used in the next pass; the
+// last cell of such a tree is placed by its network level, so that trees whose inflow comes early
+// (small levels) run before, not after, a main stem whose inflow comes late. Ranks are the chunk's
+// distinct places in order, 0 first, with up to `gap` ranks from one place to the next where the
+// levels are that far apart: with several sub-steps, an early tree then has its first sub-steps done
+// before the pass that waits for a late one. nrank is the number of ranks, at most 253.
+constexpr int SCHED_GAP = 4;
+static_assert((WAVE - 1) * SCHED_GAP + 1 <= 255, "ranks are stored in 8 bits");
+template <class Part>
+static void chunk_ranks(const int64_t n, const Part& part, const std::vector<int>& down, const std::vector<int>& level,
+                        const int gap, std::vector<uint8_t>& rank, std::vector<uint8_t>& nrank) {
+    const int64_t nch = (n + WAVE - 1) / WAVE;
+    rank.assign(n, 0);
+    nrank.assign(std::max<int64_t>(nch, 1), 0);
+    for (int64_t c = 0; c < nch; ++c) {
+        const int64_t q0 = c * WAVE, q1 = std::min<int64_t>(q0 + WAVE, n);
+        int key[WAVE], seen[WAVE], place[WAVE] = {0}, m = 0;
+        for (int64_t q = q1 - 1; q >= q0; --q) {  // downstream cells first
+            if (!part(q)) continue;
+            const int dn = down[q];
+            key[q - q0] = dn > q && dn < q1 ? key[dn - q0] - 1 : level[q];
+            seen[m++] = key[q - q0];
+        }
+        std::sort(seen, seen + m);
+        m = (int)(std::unique(seen, seen + m) - seen);
+        for (int j = 1; j < m; ++j) place[j] = place[j - 1] + std::min(seen[j] - seen[j - 1], gap);
+        for (int64_t q = q0; q < q1; ++q)
+            if (part(q)) rank[q] = (uint8_t)place[std::lower_bound(seen, seen + m, key[q - q0]) - seen];
+        nrank[c] = (uint8_t)(m > 0 ? place[m - 1] + 1 : 0);
+    }
 }
 
 extern "C" int32_t wfh_create(const wfh_config* cfg, const wfh_static* st, wfh_handle** out) {
@@ -2911,47 +2936,26 @@ extern "C" int32_t wfh_create(const wfh_config* cfg, const wfh_static* st, wfh_h
         for (size_t e = 0; e < up_idx.size(); ++e) up_f[e] = fftr[h->land_of[up_idx[e]]];
         if ((rc = put_raw<int>(h, up_ptr, D.up_ptr))) goto done;
         if ((rc = put_raw<int>(h, up_idx, D.up_idx))) goto done;
-        {  // chain chunks of the land lists (run_chain): full, at most 4 upstream cells per lane,
-           // and lane l's only upstream cell inside the chunk is lane l-1
-            const int64_t nch = (n + WAVE - 1) / WAVE;
-            std::vector<int> chain((size_t)nch, 0);
-            for (int64_t c = 0; c < nch; ++c) {
-                bool ok = (c + 1) * WAVE <= n;
-                for (int l = 0; ok && l < WAVE; ++l) {
-                    const int64_t q = c * WAVE + l;
-                    int inside = 0;
-                    ok = up_ptr[q + 1] - up_ptr[q] <= 4;
-                    for (int e = up_ptr[q]; ok && e < up_ptr[q + 1]; ++e)
-                        if (up_idx[e] / WAVE == c) {
-                            ++inside;
-                            ok = up_idx[e] == q - 1;
-                        }
-                    ok = ok && inside == (l > 0 ? 1 : 0);
-                }
-                chain[c] = ok ? 1 : 0;
+        {  // schedules of the chunks (run_sched), over all cells and over the river cells
+            std::vector<int> node_level(n), river_dn(n, -1);
+            for (int64_t q = 0; q < n; ++q) {
+                node_level[q] = level[h->land_of[q]];
+                if (flags[q] & 4) river_dn[q] = down_node[q];
             }
-            if ((rc = put_raw<int>(h, chain, D.chain_land))) goto done;
-            // the same for the river lists over the node order: every cell a river cell
-            std::vector<int> chain_r((size_t)nch, 0);
-            for (int64_t c = 0; c < nch; ++c) {
-                bool ok = (c + 1) * WAVE <= n;
-                for (int l = 0; ok && l < WAVE; ++l) {
-                    const int64_t q = c * WAVE + l;
-                    const int r = river_of[q];
-                    ok = r >= 0;
-                    if (!ok) break;
-                    int inside = 0;
-                    ok = rup_ptr[r + 1] - rup_ptr[r] <= 4;
-                    for (int e = rup_ptr[r]; ok && e < rup_ptr[r + 1]; ++e)
-                        if (rup_node[e] / WAVE == c) {
-                            ++inside;
-                            ok = rup_node[e] == q - 1;
-                        }
-                    ok = ok && inside == (l > 0 ? 1 : 0);
-                }
-                chain_r[c] = ok ? 1 : 0;
-            }
-            if ((rc = put_raw<int>(h, chain_r, D.chain_rl))) goto done;
+            double dts[2];
+            const bool one = adaptive || fp || linked;  // one sub-step per launch
+            const bool land_many = !one && (sub_steps(cfg->dt, cfg->subsurface_dt, dts) > 1 ||
+                                            sub_steps(cfg->dt, cfg->land_dt, dts) > 1);
+            const bool river_many = !one && sub_steps(cfg->dt, cfg->river_dt, dts) > 1;
+            const auto all = [](int64_t) { return true; };
+            const auto riv = [&](int64_t q) { return river_of[q] >= 0; };
+            std::vector<uint8_t> rank, nrank;
+            chunk_ranks(n, all, down_node, node_level, land_many ? SCHED_GAP : 1, rank, nrank);
+            if ((rc = put_raw<uint8_t>(h, rank, D.rank_land))) goto done;
+            if ((rc = put_raw<uint8_t>(h, nrank, D.nrank_land))) goto done;
+            chunk_ranks(n, riv, river_dn, node_level, river_many ? SCHED_GAP : 1, rank, nrank);
+            if ((rc = put_raw<uint8_t>(h, rank, D.rank_riv))) goto done;
+            if ((rc = put_raw<uint8_t>(h, nrank, D.nrank_riv))) goto done;
         }
         if ((rc = put_raw<double>(h, up_f, D.up_f))) goto done;
         if ((rc = put_raw<int>(h, river_of, D.river_of))) goto done;
@@ -2984,26 +2988,6 @@ extern "C" int32_t wfh_create(const wfh_config* cfg, const wfh_static* st, wfh_h
             }
             if ((rc = put_raw<int>(h, sup_ptr, D.sup_ptr))) goto done;
             if ((rc = put_raw<int>(h, sup_idx, D.sup_idx))) goto done;
-            {  // chain chunks of these lists (run_chain), as for the land lists
-                const int64_t nch = (n + WAVE - 1) / WAVE;
-                std::vector<int> chain((size_t)nch, 0);
-                for (int64_t c = 0; c < nch && D.snow_lat; ++c) {
-                    bool ok = (c + 1) * WAVE <= n;
-                    for (int l = 0; ok && l < WAVE; ++l) {
-                        const int64_t q = c * WAVE + l;
-                        int inside = 0;
-                        ok = sup_ptr[q + 1] - sup_ptr[q] <= 4;
-                        for (int e = sup_ptr[q]; ok && e < sup_ptr[q + 1]; ++e)
-                            if (sup_idx[e] / WAVE == c) {
-                                ++inside;
-                                ok = sup_idx[e] == q - 1;
-                            }
-                        ok = ok && inside == (l > 0 ? 1 : 0);
-                    }
-                    chain[c] = ok ? 1 : 0;
-                }
-                if ((rc = put_raw<int>(h, chain, D.chain_sup))) goto done;
-            }
             if ((rc = put_state(h, {}, D.snow_in))) goto done;
             if ((rc = put_state(h, {}, D.snow_out))) goto done;
         }
@@ -3352,25 +3336,13 @@ extern "C" int32_t wfh_create(const wfh_config* cfg, const wfh_static* st, wfh_h
                 if ((rc = put_raw<int>(h, si, X.fp_sup_idx))) goto done;
             }
             X.nchunks_r = (int)((nriv + WAVE - 1) / WAVE);
-            {  // chain chunks (run_chain): full, at most 4 upstream cells per lane, and lane l's only
-               // upstream cell inside the chunk is lane l-1
-                std::vector<int> chain((size_t)std::max(X.nchunks_r, 1), 0);
-                for (int c = 0; c < X.nchunks_r; ++c) {
-                    bool ok = (int64_t)(c + 1) * WAVE <= nriv;
-                    for (int l = 0; ok && l < WAVE; ++l) {
-                        const int p = c * WAVE + l;
-                        int inside = 0;
-                        ok = rp_ptr[p + 1] - rp_ptr[p] <= 4;
-                        for (int e = rp_ptr[p]; ok && e < rp_ptr[p + 1]; ++e)
-                            if (rp_idx[e] / WAVE == c) {
-                                ++inside;
-                                ok = rp_idx[e] == p - 1;
-                            }
-                        ok = ok && inside == (l > 0 ? 1 : 0);
-                    }
-                    chain[c] = ok ? 1 : 0;
-                }
-                if ((rc = put_raw<int>(h, chain, X.chain_r))) goto done;
+            {  // schedules of the chunks of river positions (run_sched)
+                std::vector<int> rp_level(nriv);
+                for (int64_t k = 0; k < nriv; ++k) rp_level[k] = level[h->river_land[rp_r[k]]];
+                std::vector<uint8_t> rank, nrank;
+                chunk_ranks(nriv, [](int64_t) { return true; }, rp_down, rp_level, 1, rank, nrank);
+                if ((rc = put_raw<uint8_t>(h, rank, X.rank_r))) goto done;
+                if ((rc = put_raw<uint8_t>(h, nrank, X.nrank_r))) goto done;
             }
             hipError_t ea = hipSuccess, eb;
             X.szi = dalloc<double>(h, n, eb); if (eb != hipSuccess) ea = eb;
