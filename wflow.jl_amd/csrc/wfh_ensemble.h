@@ -27,6 +27,19 @@ constexpr int ENS_PRE = 10;          // fluxes of the vertical update that the r
 // the pre-buffer), or the routing only (the column taken from the pre-buffer).
 enum { ENS_FUSED = 0, ENS_COLUMN = 1, ENS_ROUTE = 2 };
 
+constexpr int ENS_CHAIN_UP = 4;  // upstream cells of a record
+// What a cell of a chain stage reads, in the order of the strands (index: the cell's pre-buffer
+// slot), so that a wave loads the next cells' records and values without chasing indexes: node,
+// river cell (or -1), first edge and number of edges of the land and the river network, position
+// among them of the cell before it in the strand (or -1), and the other upstream cells (an unused
+// entry and the one before it in the strand hold the cell itself: a harmless address).
+struct alignas(16) EnsRec {
+    int v, r;
+    int e0, deg, in, up[ENS_CHAIN_UP];
+    int re0, rdeg, rin, rup[ENS_CHAIN_UP];
+};
+static_assert(sizeof(EnsRec) == 64, "a record is one scalar load");
+
 struct EnsDev {
     int n, nriv, M, G;  // cells, river cells, members, member groups of 64
     double dt;
@@ -58,6 +71,7 @@ struct EnsDev {
     // the vertical update of chain-stage cells, done beforehand in a parallel pass: node -> slot
     // (or -1), and the fluxes the routing part reads, [ENS_PRE][npre * M]
     const int* pre_slot;
+    const EnsRec* rec;
     double* pre;
     size_t pre_stride;
     // learned warm start of the kinematic-wave solves (LEARN instantiation): the network, and the
@@ -484,6 +498,303 @@ __global__ void __launch_bounds__(256, 2) k_ens_stage(EnsDev e, int s0, int ns) 
     }
 }
 
+// ---- chain stages, pipelined over the families ----------------------------------------------
+// A chain stage is a serial walk down its strands, and near the outlet there are few of them: its
+// time is the latency of one cell times the cells of a strand. One wave per strand and member group
+// (k_ens_stage) does a cell's subsurface, overland and river sub-steps one after another, with the
+// cell's loads in front. Here a block of 2 + S_r waves walks a strand, one family (river sub-step)
+// per wave: in round t the subsurface wave does cell t, the overland wave cell t - 1, river sub-step
+// k cell t - 2 - k. A family's inflow from the cell above is the wave's own result of the round
+// before (a register); what a cell hands to its next family goes through LDS, in two buffers by the
+// parity of the round, with one barrier a round. Values that do not depend on the strand (states,
+// parameters, inflow from other strands) are loaded one round ahead, their addresses (EnsRec) two.
+// Operations and their order are ens_cell's. Measured, 128 members of 257 x 251 cells (308 levels, 285 of
+// them in such stages): three steps 18.6 -> 11.6 ms; a cell of the main stem took 16 us, a round takes
+// 8 us, set by the overland wave, whose solves take up to 126 updates where a member's cell is dry.
+constexpr int ENS_CHAIN_SR = 6;  // river sub-steps at most: 8 waves a block, 256 registers each
+enum { ENS_X_INWATER = 0, ENS_X_TOR, ENS_X_RQLAT, ENS_X_RIVER, ENS_X = ENS_X_RIVER + 3 * (ENS_CHAIN_SR - 1) };
+typedef double EnsXchg[2][ENS_X][WAVE];
+
+// Inflow of one family of one cell: values and fractions of the first ENS_CHAIN_UP edges.
+struct EnsUp {
+    double q[ENS_CHAIN_UP], f[ENS_CHAIN_UP];
+    __device__ __forceinline__ void load(const EnsDev& e, const EnsRec& r, const double* src, const int m) {
+#pragma unroll
+        for (int j = 0; j < ENS_CHAIN_UP; ++j) {
+            q[j] = src[(size_t)r.up[j] * e.M + m];
+            f[j] = j < r.deg ? e.up_f[r.e0 + j] : 0.0;
+        }
+    }
+    // left fold in ascending upstream id; last: the strand's own value
+    __device__ __forceinline__ void fold(const EnsDev& e, const EnsRec& r, const double* src, const int m,
+                                         const double last, double& qin, double& tor) const {
+        qin = 0.0;
+        tor = 0.0;
+#pragma unroll
+        for (int j = 0; j < ENS_CHAIN_UP; ++j)
+            if (j < r.deg) {
+                const double qu = j == r.in ? last : q[j];
+                qin = qin + qu * (1.0 - f[j]);
+                tor = tor + qu * f[j];
+            }
+        for (int j = ENS_CHAIN_UP; j < r.deg; ++j) {
+            const double qu = j == r.in ? last : src[(size_t)e.up_idx[r.e0 + j] * e.M + m];
+            const double fu = e.up_f[r.e0 + j];
+            qin = qin + qu * (1.0 - fu);
+            tor = tor + qu * fu;
+        }
+    }
+};
+
+template <int N>
+struct EnsChainLand {
+    double us[N], zi, recharge, sat_exc, rl, inf_exc, aol, nrr, aet, leak, store_prev;
+    double sq0, qmax, canopy, ss, sw;
+    double P, kv0, fk, khf, area, flen, fw, slope, sy, ts, tr, dsoil, tfc;
+    EnsUp up;
+    __device__ __forceinline__ void load(const EnsDev& e, const EnsRec& r, const int slot, const int m) {
+        const int v = r.v;
+        const size_t M = (size_t)e.M, i = (size_t)v * M + m, nM = (size_t)e.n * M, ps = e.pre_stride;
+        const double* q = e.pre + (size_t)slot * M + m;
+#pragma unroll
+        for (int k = 0; k < N; ++k) us[k] = e.ustore[k * nM + i];
+        zi = q[0], recharge = q[ps], sat_exc = q[2 * ps], rl = q[3 * ps], inf_exc = q[4 * ps], aol = q[5 * ps];
+        nrr = q[6 * ps], aet = q[7 * ps], leak = q[8 * ps], store_prev = q[9 * ps];
+        sq0 = e.ssf_q[i], qmax = e.qmax[i], canopy = e.canopy[i];
+        ss = e.snow_s[i], sw = e.snow_w[i];
+        up.load(e, r, e.ssf_q, m);
+        P = e.P[v], kv0 = ens_ld(e.kv0, v), fk = ens_ld(e.f, v), khf = ens_ld(e.khfrac, v), area = ens_ld(e.area, v);
+        flen = ens_ld(e.fl, v), fw = ens_ld(e.fw, v), slope = ens_ld(e.slope, v), sy = ens_ld(e.sy, v);
+        ts = ens_ld(e.ts, v), tr = ens_ld(e.tr, v), dsoil = ens_ld(e.d, v), tfc = ens_ld(e.tfc, v);
+    }
+};
+
+// The subsurface wave; returns the largest |land balance error| of its cells.
+template <int N>
+__device__ __forceinline__ double ens_chain_land(const EnsDev& e, EnsXchg& X, const int base, const int len,
+                                                 const int rounds, const int lane, const int m) {
+    const size_t nM = (size_t)e.n * e.M;
+    const double dt = e.dt, fa = e.fa[m], fb = e.fb[m];
+    double worst = 0.0, last = 0.0;
+    EnsRec rn = e.rec[base], r2 = e.rec[base + (len > 1 ? 1 : 0)];
+    EnsChainLand<N> nx;
+    nx.load(e, rn, base, m);
+    for (int t = 0; t < rounds; ++t) {
+        if (t < len) {
+            const EnsChainLand<N> c = nx;
+            const EnsRec rc = rn;
+            if (t + 1 < len) {
+                rn = r2;
+                nx.load(e, rn, base + t + 1, m);
+                if (t + 2 < len) r2 = e.rec[base + t + 2];
+            }
+            asm volatile("" ::: "memory");  // (the loads ahead stay here)
+            const size_t i = (size_t)rc.v * e.M + m;
+            const double kv0 = c.kv0 * fa, fk = c.fk * fb;
+            const double kh0 = c.khf * kv0;
+            Column<N> col;
+            soil_layers<N>(c.dsoil, e.cfg_cum, e.cfg_thick, col.act, col.cum);
+#pragma unroll
+            for (int k = 0; k < N; ++k) col.ustore[k] = c.us[k];
+            col.zi = c.zi;
+            col.n_unsat = set_layerthickness<N>(col.zi, col.cum, col.act, col.thick);
+            col.theta_e = c.ts - c.tr;
+            col.theta_fc_r = c.tfc - c.tr;
+            double qin, tor;
+            c.up.fold(e, rc, e.ssf_q, m, last, qin, tor);
+            const SsfPrep pp = ssf_prepare(c.sq0, col.zi, c.slope, c.sy, dt, c.flen, kh0, fk, INFINITY);
+            double flx = c.recharge * c.area;  // flux!(::RechargeModel) with check_flux
+            if (col.zi >= c.dsoil) flx = wfh_max(0.0, flx);
+            const double qnb = 0.0 + flx;
+            double qn, zin, exf, net;
+            const double z0 = col.zi;
+            if (kinematic_wave_ssf<N>(qin, c.sq0, z0, qnb, c.slope, c.sy, c.dsoil, dt, c.flen, c.fw, c.qmax, kh0, fk,
+                                      INFINITY, pp, col, true, qn, zin, exf, net))
+                update_ustorelayerdepth<N>(col, z0, zin);
+            last = qn;
+            e.ssf_q[i] = qn;
+            const double s_exf_avg = (0.0 + exf * dt) / dt, s_qin_avg = (0.0 + qin * dt) / dt;
+            const double s_q_avg = (0.0 + qn * dt) / dt, s_tor_avg = (0.0 + tor * dt) / dt;
+            double usd = 0.0;
+            bool first = true;
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+                if (k < col.n_unsat) {
+                    usd = first ? col.ustore[k] : usd + col.ustore[k];
+                    first = false;
+                }
+            const double sbm_runoff = wfh_max(0.0, s_exf_avg + c.sat_exc + c.rl + c.inf_exc);
+            const double swd = (c.dsoil - col.zi) * (c.ts - c.tr);
+            const double net_runoff = sbm_runoff - c.aol;
+            X[t & 1][ENS_X_INWATER][lane] = (net_runoff + 0.0) * c.area + 0.0;
+            X[t & 1][ENS_X_TOR][lane] = s_tor_avg;
+#pragma unroll
+            for (int k = 0; k < N; ++k) e.ustore[k * nM + i] = col.ustore[k];
+            e.swd[i] = swd;
+            e.tsws[i] = swd + usd;
+            if (e.balance) {  // land balance  mass_balance.jl:215-253
+                const double t_in = s_qin_avg / c.area + (c.P + 0.0) + 0.0 + 0.0 / c.area;
+                const double vout = net_runoff + c.aet + c.nrr + c.leak + 0.0;
+                const double t_out = s_q_avg / c.area + vout + 0.0 + 0.0 / c.area;
+                const double snow_bal = e.snow ? c.ss + c.sw : 0.0 + 0.0;
+                const double storage = (swd + usd) + c.canopy + snow_bal + 0.0 * 0.0 + 0.0;
+                const double rate = (storage - c.store_prev) / dt;
+                worst = wfh_max(worst, wfh_fabs(t_in - t_out - rate));
+            }
+        }
+        __syncthreads();
+    }
+    return worst;
+}
+
+struct EnsChainOverland {
+    double oq0, alpha, nrr, area, flen, sfw, rfl, rarea;
+    EnsUp up;
+    __device__ __forceinline__ void load(const EnsDev& e, const EnsRec& r, const int slot, const int m) {
+        const int v = r.v, rr = r.r >= 0 ? r.r : 0;
+        const size_t i = (size_t)v * e.M + m;
+        oq0 = e.ol_q[i], alpha = e.alpha[i], nrr = e.pre[6 * e.pre_stride + (size_t)slot * e.M + m];
+        up.load(e, r, e.ol_q, m);
+        area = ens_ld(e.area, v), flen = ens_ld(e.fl, v), sfw = ens_ld(e.sfw, v);
+        rfl = r.r >= 0 ? e.r_fl[rr] : 1.0, rarea = r.r >= 0 ? e.r_area[rr] : 0.0;
+    }
+};
+
+__device__ __forceinline__ void ens_chain_overland(const EnsDev& e, EnsXchg& X, const int base, const int len,
+                                                   const int rounds, const int lane, const int m) {
+    const double dt = e.dt;
+    double last = 0.0;
+    EnsRec rn = e.rec[base], r2 = e.rec[base + (len > 1 ? 1 : 0)];
+    EnsChainOverland nx;
+    nx.load(e, rn, base, m);
+    for (int t = 0; t < rounds; ++t) {
+        const int c0 = t - 1;
+        if (c0 >= 0 && c0 < len) {
+            const EnsChainOverland c = nx;
+            const EnsRec rc = rn;
+            if (c0 + 1 < len) {
+                rn = r2;
+                nx.load(e, rn, base + c0 + 1, m);
+                if (c0 + 2 < len) r2 = e.rec[base + c0 + 2];
+            }
+            asm volatile("" ::: "memory");
+            const size_t i = (size_t)rc.v * e.M + m;
+            const double o_inwater = X[(t - 1) & 1][ENS_X_INWATER][lane];
+            const double s_tor_avg = X[(t - 1) & 1][ENS_X_TOR][lane];
+            double qin_all, tor;  // surface_kinwave.jl:317-326
+            c.up.fold(e, rc, e.ol_q, m, last, qin_all, tor);
+            const double oqlat = o_inwater / c.flen;
+            const KwPrep op = kw_prepare(c.oq0, oqlat, c.alpha, dt, c.flen);
+            double qin = 0.0;
+            if (c.sfw > 0.0) qin = qin_all;
+            double qn, ar;
+            kw_solve(qin, op, c.alpha, qn, ar);
+            last = qn;
+            e.ol_q[i] = qn;
+            if (c.sfw > 0.0) e.ol_h[i] = ar / c.sfw;  // (unchanged otherwise)
+            const double o_tor_avg = (0.0 + tor * dt) / dt;
+            if (rc.r >= 0) {
+                const double r_inwater = (s_tor_avg + o_tor_avg + c.nrr * c.area) + 0.0 * c.rarea;
+                const double rqlat = r_inwater / c.rfl;
+                double inflow = 0.0 / c.rfl;
+                inflow -= 0.0 / c.rfl;
+                X[t & 1][ENS_X_RQLAT][lane] = rqlat + inflow;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+struct EnsChainRiver {
+    double q0, alpha, rfl, rfw, q[ENS_CHAIN_UP];
+    __device__ __forceinline__ void load(const EnsDev& e, const EnsRec& r, const double* src, const int m) {
+        if (r.r < 0) return;
+        const size_t ri = (size_t)r.r * e.M + m;
+        q0 = e.r_q[ri], alpha = e.r_alpha[ri];
+#pragma unroll
+        for (int j = 0; j < ENS_CHAIN_UP; ++j) q[j] = src[(size_t)r.rup[j] * e.M + m];
+        rfl = e.r_fl[r.r], rfw = e.r_fw[r.r];
+    }
+};
+
+// River sub-step k.
+__device__ __forceinline__ void ens_chain_river(const EnsDev& e, EnsXchg& X, const int base, const int len,
+                                                const int rounds, const int lane, const int m, const int k) {
+    const size_t rM = (size_t)e.nriv * e.M;
+    const bool final_step = k == e.S_r - 1;
+    double* qk = final_step ? e.r_q : e.rq_sub + (size_t)k * rM;
+    const double dts = e.dts_r[final_step ? 1 : 0];
+    double last = 0.0;
+    EnsRec rn = e.rec[base], r2 = e.rec[base + (len > 1 ? 1 : 0)];
+    EnsChainRiver nx{};
+    nx.load(e, rn, qk, m);
+    for (int t = 0; t < rounds; ++t) {
+        const int c0 = t - 2 - k;
+        if (c0 >= 0 && c0 < len) {
+            const EnsChainRiver c = nx;
+            const EnsRec rc = rn;
+            if (c0 + 1 < len) {
+                rn = r2;
+                nx.load(e, rn, qk, m);
+                if (c0 + 2 < len) r2 = e.rec[base + c0 + 2];
+            }
+            asm volatile("" ::: "memory");
+            if (rc.r >= 0) {
+                const size_t ri = (size_t)rc.r * e.M + m;
+                const double(*x)[WAVE] = X[(t - 1) & 1];
+                const double rqlat = x[k == 0 ? (int)ENS_X_RQLAT : ENS_X_RIVER + 3 * (k - 1) + 2][lane];
+                const double rq = k == 0 ? c.q0 : x[ENS_X_RIVER + 3 * (k - 1)][lane];
+                const double cum = k == 0 ? 0.0 : x[ENS_X_RIVER + 3 * (k - 1) + 1][lane];
+                double sumq = 0.0;  // surface_kinwave.jl:520
+#pragma unroll
+                for (int j = 0; j < ENS_CHAIN_UP; ++j)
+                    if (j < rc.rdeg) sumq = sumq + (j == rc.rin ? last : c.q[j]);
+                for (int j = ENS_CHAIN_UP; j < rc.rdeg; ++j)
+                    sumq = sumq + (j == rc.rin ? last : qk[(size_t)e.rup_idx[rc.re0 + j] * e.M + m]);
+                const KwPrep rp = kw_prepare(rq, rqlat, c.alpha, dts, c.rfl);
+                const double qin = 0.0 + sumq;
+                double qn, ar;
+                kw_solve(qin, rp, c.alpha, qn, ar);
+                last = qn;
+                const double r_q_cum = cum + qn * dts;
+                qk[ri] = qn;
+                if (final_step) {
+                    e.r_h[ri] = ar / c.rfw;
+                    e.r_storage[ri] = c.rfl * ar;
+                    e.r_q_avg[ri] = r_q_cum / e.dt;
+                } else {
+                    double(*y)[WAVE] = X[t & 1];
+                    y[ENS_X_RIVER + 3 * k][lane] = qn;
+                    y[ENS_X_RIVER + 3 * k + 1][lane] = r_q_cum;
+                    y[ENS_X_RIVER + 3 * k + 2][lane] = rqlat;
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// One block of 2 + S_r waves per strand and member group (S_r <= ENS_CHAIN_SR). Every wave takes
+// the same number of barriers.
+template <int N>
+__global__ void __launch_bounds__(64 * (2 + ENS_CHAIN_SR)) k_ens_chain(EnsDev e, int s0) {
+    __shared__ EnsXchg X;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int st = s0 + blockIdx.x / e.G, m = (blockIdx.x % e.G) * WAVE + lane;
+    const int c0 = e.strand_ptr[st], len = e.strand_ptr[st + 1] - c0;
+    const int base = e.pre_slot[e.strand_cell[c0]];  // slots run along the strand
+    const int rounds = len + 1 + e.S_r;
+    if (w == 0) {
+        const double worst = ens_chain_land<N>(e, X, base, len, rounds, lane, m);
+        if (e.balance && worst > 0.0) atomicMax(&e.bal_max[m], (unsigned long long)wfh_bits(worst));
+    } else if (w == 1) {
+        ens_chain_overland(e, X, base, len, rounds, lane, m);
+    } else {
+        ens_chain_river(e, X, base, len, rounds, lane, m, w - 2);
+    }
+}
+
 __global__ void k_ens_zero_u64(unsigned long long* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0ull;
@@ -575,6 +886,7 @@ struct EnsSchedule {
     int* d_ptr = nullptr;
     int* d_cell = nullptr;
     int* d_pre_slot = nullptr;
+    EnsRec* d_rec = nullptr;  // [npre]
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     double ms = -1.0;  // measured step time (autotuner)
@@ -590,6 +902,7 @@ struct wfh_ensemble {
     std::vector<std::vector<int>> ups;        // node -> upstream nodes
     std::vector<int> down;                    // node -> downstream node or -1
     int max_level = 0;
+    std::vector<int> up_ptr, up_idx, rup_ptr, rup_idx, river_of;  // the device's edges, for EnsRec
     std::vector<EnsSchedule> cand;            // schedules (the autotuner's candidates)
     double* pre = nullptr;                    // pre-buffer shared by the schedules, [ENS_PRE][pre_cap * M]
     int pre_cap = 0;
@@ -713,12 +1026,53 @@ void ens_build_schedule(const wfh_ensemble* x, EnsSchedule& s) {
     }
 }
 
+// A chain stage is pipelined over the families (k_ens_chain) when its blocks all run at once, one
+// per CU (six to eight waves of up to 256 registers each). With more strands the GPU has work for
+// every wave anyway, and the pipeline's waiting waves would only hold slots.
+constexpr int64_t ENS_CHAIN_BLOCKS = 256;
+
+// The records of the chain stages' cells, by slot.
+std::vector<EnsRec> ens_records(const wfh_ensemble* x, const EnsSchedule& s) {
+    std::vector<EnsRec> rec(s.npre);
+    const auto edges = [](const std::vector<int>& ptr, const std::vector<int>& idx, int cell, int before, int& e0,
+                          int& deg, int& in, int* up) {
+        e0 = ptr[cell];
+        deg = ptr[cell + 1] - e0;
+        in = -1;
+        for (int j = 0; j < ENS_CHAIN_UP; ++j) up[j] = cell;
+        for (int j = 0; j < deg; ++j) {
+            if (before >= 0 && idx[e0 + j] == before)
+                in = j;
+            else if (j < ENS_CHAIN_UP)
+                up[j] = idx[e0 + j];
+        }
+    };
+    for (size_t k = 0; k < s.stages.size(); ++k) {
+        if (s.modes[k] != ENS_ROUTE) continue;
+        for (int t = s.stages[k].first; t < s.stages[k].first + s.stages[k].second; ++t)
+            for (int c = s.strand_ptr[t]; c < s.strand_ptr[t + 1]; ++c) {
+                const int v = s.strand_cell[c], r = x->river_of[v];
+                const int before = c > s.strand_ptr[t] ? s.strand_cell[c - 1] : -1;
+                EnsRec& q = rec[s.pre_slot[v]];
+                q = EnsRec{};
+                q.v = v;
+                q.r = r;
+                edges(x->up_ptr, x->up_idx, v, before, q.e0, q.deg, q.in, q.up);
+                q.rin = -1;
+                if (r >= 0)
+                    edges(x->rup_ptr, x->rup_idx, r, before >= 0 ? x->river_of[before] : -1, q.re0, q.rdeg, q.rin, q.rup);
+            }
+    }
+    return rec;
+}
+
 template <int N>
 void ens_launch_stages(wfh_ensemble* x, const EnsSchedule& s, hipStream_t st) {
     EnsDev e = x->e;
     e.strand_ptr = s.d_ptr;
     e.strand_cell = s.d_cell;
     e.pre_slot = s.d_pre_slot;
+    e.rec = s.d_rec;
     e.pre = x->pre;
     e.pre_stride = (size_t)x->pre_cap * x->M;
     if (e.balance) hipLaunchKernelGGL(k_ens_zero_u64, dim3((x->M + 255) / 256), dim3(256), 0, st, e.bal_max, x->M);
@@ -730,7 +1084,10 @@ void ens_launch_stages(wfh_ensemble* x, const EnsSchedule& s, hipStream_t st) {
         const int var = e.mlp ? ENS_LEARN : (e.kw_hist || e.harvest) ? ENS_INSTR : ENS_PLAIN;
         if (s.modes[k] == ENS_COLUMN)
             hipLaunchKernelGGL((k_ens_stage<N, ENS_COLUMN, ENS_PLAIN>), grid, block, 0, st, e, sg.first, sg.second);
-        else if (s.modes[k] == ENS_ROUTE) {
+        else if (s.modes[k] == ENS_ROUTE && var == ENS_PLAIN && e.S_r <= ENS_CHAIN_SR &&
+                 (int64_t)sg.second * e.G <= ENS_CHAIN_BLOCKS) {
+            hipLaunchKernelGGL(k_ens_chain<N>, dim3(sg.second * e.G), dim3(WAVE * (2 + e.S_r)), 0, st, e, sg.first);
+        } else if (s.modes[k] == ENS_ROUTE) {
             auto kr = var == ENS_LEARN   ? k_ens_stage<N, ENS_ROUTE, ENS_LEARN>
                       : var == ENS_INSTR ? k_ens_stage<N, ENS_ROUTE, ENS_INSTR>
                                          : k_ens_stage<N, ENS_ROUTE, ENS_PLAIN>;
@@ -752,7 +1109,10 @@ int32_t ens_prepare(wfh_ensemble* x, EnsSchedule& s) {
         s.d_ptr = ealloc<int>(x, s.strand_ptr.size());
         s.d_cell = ealloc<int>(x, s.strand_cell.size());
         s.d_pre_slot = ealloc<int>(x, s.pre_slot.size());
-        if (!s.d_ptr || !s.d_cell || !s.d_pre_slot) return efail(x, WFH_ERR_HIP, "hipMalloc schedule");
+        s.d_rec = ealloc<EnsRec>(x, s.npre);
+        if (!s.d_ptr || !s.d_cell || !s.d_pre_slot || !s.d_rec) return efail(x, WFH_ERR_HIP, "hipMalloc schedule");
+        const std::vector<EnsRec> rec = ens_records(x, s);
+        EHIP(x, hipMemcpy(s.d_rec, rec.data(), rec.size() * sizeof(EnsRec), hipMemcpyHostToDevice));
         EHIP(x, hipMemcpy(s.d_pre_slot, s.pre_slot.data(), s.pre_slot.size() * sizeof(int), hipMemcpyHostToDevice));
         EHIP(x, hipMemcpy(s.d_ptr, s.strand_ptr.data(), s.strand_ptr.size() * sizeof(int), hipMemcpyHostToDevice));
         EHIP(x, hipMemcpy(s.d_cell, s.strand_cell.data(), s.strand_cell.size() * sizeof(int),
@@ -899,6 +1259,14 @@ extern "C" int32_t wfh_ens_create(const wfh_config* cfg, const wfh_static* st, i
         x->level[q] = lv;
         x->max_level = std::max(x->max_level, lv);
     }
+    const auto read = [](std::vector<int>& v, const int* d, size_t count) {
+        v.resize(count);
+        return count == 0 || hipMemcpy(v.data(), d, count * sizeof(int), hipMemcpyDeviceToHost) == hipSuccess;
+    };
+    if (!read(x->up_ptr, e.up_ptr, n + 1) || !read(x->up_idx, e.up_idx, x->up_ptr[n]) ||
+        !read(x->river_of, e.river_of, n) || !read(x->rup_ptr, e.rup_ptr, nriv > 0 ? nriv + 1 : 0) ||
+        !read(x->rup_idx, e.rup_idx, nriv > 0 ? x->rup_ptr[nriv] : 0))
+        return bail(WFH_ERR_HIP, "ensemble: reading the base model's topology");
     const size_t nM = (size_t)n * M, rM = (size_t)std::max(nriv, 1) * M;
     double** big[] = {&e.canopy, &e.snow_s, &e.snow_w, &e.tsoil, &e.swd, &e.tsws, &e.ssf_q, &e.ol_q, &e.ol_h};
     for (double** pp : big)
