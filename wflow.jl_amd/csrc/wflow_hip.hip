@@ -185,6 +185,7 @@ struct RouteArgs {
     long spin_limit;  // SPIN_LIMIT (wfh_test_route_stall lowers it)
     int parity;
     int nchunks;
+    int land_only;  // the river follows in launches of its own (floodplain, linked weirs)
     // multi-step run (k_route<N, false, true>): steps of the launch, per chunk the number of its
     // steps completed, the forcing frames of the steps ([nsteps][n], node order) and optionally
     // each step's river discharge average ([nsteps][nriv], river order)
@@ -1380,6 +1381,8 @@ __global__ void __launch_bounds__(ROUTE_BLOCK) __attribute__((amdgpu_waves_per_e
         if (valid)
             r_inwater = ol_finish<MULTI>(d, p, r, ol.q, oh, o_storage, ol.qin, ol.q_cum, o_tor_cum, ol.qin_cum, o_inwater,
                                          o_store_prev, s_tor_avg, nrr, area, rarea);
+        if constexpr (EXT && !MULTI && !FUSE)
+            if (a.land_only) continue;
 
         // ---------------- river kinematic wave ----------------
         const bool rcons_in = riv && (fl & 4) && cons_in;  // a river cell drains to the land downstream
@@ -3101,7 +3104,7 @@ extern "C" int32_t wfh_create(const wfh_config* cfg, const wfh_static* st, wfh_h
             }
             double dts[2];
             const bool one = adaptive || fp || linked;  // one sub-step per launch
-            const bool land_many = !one && (sub_steps(cfg->dt, cfg->subsurface_dt, dts) > 1 ||
+            const bool land_many = !adaptive && (sub_steps(cfg->dt, cfg->subsurface_dt, dts) > 1 ||
                                             sub_steps(cfg->dt, cfg->land_dt, dts) > 1);
             const bool river_many = !one && sub_steps(cfg->dt, cfg->river_dt, dts) > 1;
             const auto all = [](int64_t) { return true; };
@@ -3697,16 +3700,29 @@ static int32_t launch_adaptive(wfh_handle* h) {
         return a;
     };
     int32_t rc;
-    // subsurface: the water table handed over by the soil (sbm_model.jl:74-81)
-    HIPCHK(h, hipMemcpyAsync(h->ad.szi, h->d.zi, (size_t)n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
-    for (int fam = 0; fam < 3; ++fam) {
+    const bool adaptive = h->cfg.kinematic_wave_adaptive != 0;
+    if (!adaptive) {
+        // Fixed sub-steps (a floodplain model, linked weirs): subsurface and overland flow need nothing
+        // of the river, so all their sub-steps run in one launch, one walk down the network.
+        // Two hourly steps of 509 x 503 cells with a floodplain: 6.81 -> 6.04 ms against a launch per family.
+        RouteArgs a = args();
+        a.land_only = 1;
+        hipLaunchKernelGGL((k_route<N, true>), dim3(h->route_grid), dim3(ROUTE_BLOCK), 0, h->stream, h->d, a);
+        HIPCHK(h, hipGetLastError());
+        h->nsub[0] = h->S_s;
+        h->nsub[1] = h->S_l;
+    } else {
+        // subsurface: the water table handed over by the soil (sbm_model.jl:74-81)
+        HIPCHK(h, hipMemcpyAsync(h->ad.szi, h->d.zi, (size_t)n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    }
+    for (int fam = adaptive ? 0 : 2; fam < 3; ++fam) {
         double t = 0.0;
         int k = 0;
         while (t < dt) {
             double dts;
             rc = WFH_OK;
-            if (!h->cfg.kinematic_wave_adaptive)  // fixed sub-steps (a floodplain model)
-                dts = fam == 0 ? h->cfg.subsurface_dt : fam == 1 ? h->cfg.land_dt : h->cfg.river_dt;
+            if (!adaptive)
+                dts = h->cfg.river_dt;
             else if (fam == 0)
                 rc = ssf_stable_timestep(h, dts);
             else if (fam == 1)
