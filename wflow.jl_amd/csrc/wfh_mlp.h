@@ -137,7 +137,7 @@ __device__ __noinline__ float mlp_forward_call(const MlpOps* W, float x0, float 
 // four tiles run side by side, the products over the samples are split by quadrant of W2 (one per
 // wave, samples in ascending order), and a unit's sum over the samples is a left fold by one lane
 // over a row in LDS, the order in which LDS atomics of one wave would add.
-// Measured: an epoch of 300,000 rows in minibatches of 8192 5.10 -> 0.84 ms (17.8 us for this kernel
+// Measured: an epoch of 300,000 rows in minibatches of 8192 5.10 -> 0.81 ms (17 us for this kernel
 // and 4.7 us for the Adam step a minibatch; one wave with four tiles in a row and LDS atomics per unit,
 // an Adam step, a layout launch and a read-back of the loss took 138 us). Bound by latency: 32 of 256
 // CUs have work.
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const MlpOps* __restrict__ Wp,
     // sums over the samples: dw3 (wave 0), db2 (wave 1), one unit per lane; db3 and the loss (wave 2)
     if (wave == 0) {
         float acc = 0.0f;
-#pragma unroll 4
+#pragma unroll 16
         for (int s = 0; s < MLP_GS; s += 4) {
             const float4 z = *reinterpret_cast<const float4*>(&F[lane][s]);
             const float4 d = *reinterpret_cast<const float4*>(&DY[s]);
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const MlpOps* __restrict__ Wp,
     } else if (wave == 1) {
         const float w3 = W.w3[h][(lane >> 2) & 1][4 * ((lane & 31) >> 3) + (lane & 3)];
         float acc = 0.0f;
-#pragma unroll 4
+#pragma unroll 16
         for (int s = 0; s < MLP_GS; s += 4) {
             const float4 z = *reinterpret_cast<const float4*>(&F[lane][s]);
             const float4 d = *reinterpret_cast<const float4*>(&DY[s]);
@@ -290,7 +290,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const MlpOps* __restrict__ Wp,
             if (col < 8) P[MLP_OW1 + mlp_dunit(wave, h, r) * MLP_IN + col] = g[r];
     } else if (wave == 2) {
         float acc = 0.0f;
-#pragma unroll 4
+#pragma unroll 16
         for (int s = 0; s < MLP_GS; s += 4) {
             const float4 g = *reinterpret_cast<const float4*>(&F[lane][s]);
             acc += g.x;
