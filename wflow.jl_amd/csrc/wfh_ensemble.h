@@ -1384,8 +1384,8 @@ extern "C" int32_t wfh_ens_set_forcing(wfh_ensemble* x, const double* P, const d
             EHIP(x, hipStreamSynchronize(s));
         }
     } else if (memkind == WFH_MEM_DEVICE) {
-        for (int k = 0; k < 3; ++k)
-            hipLaunchKernelGGL(k_gather, dim3((n + 255) / 256), dim3(256), 0, s, dst[k], src[k], x->base->d_land_of, n);
+        hipLaunchKernelGGL(k_gather3, dim3((n + 255) / 256), dim3(256), 0, s, dst[0], dst[1], dst[2], P, E, T,
+                           x->base->d_land_of, n);
         EHIP(x, hipGetLastError());
     } else if (memkind == WFH_MEM_DEVICE_NODE_ORDER) {
         for (int k = 0; k < 3; ++k)
