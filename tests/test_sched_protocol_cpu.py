@@ -9,7 +9,9 @@ becomes visible late.
     four, cells with up to nine upstream cells (the inbox has places for four), solves that end
     late, and chunks of which only some cells take part.
   - A cell of a chunk has the rank next above its upstream cells of the chunk.
-  - A wait that is never met ends by the spin limit, and nothing but right values has been published.
+  - A wait that is never met (of an edge with a place in the inbox, or of one beyond) ends by the spin
+    limit, and nothing but right values has been published, by no wave: one that has given up, or
+    was told to, has not passed on what it computed without its inflow.
   - The check is not vacuous: tickets in the reverse order do not drain, and wrong ranks are seen.
 """
 import ctypes
@@ -180,10 +182,11 @@ def _edges(net, place):
 
 
 @pytest.mark.parametrize("fold,ring,S", [(SSF, 4, 1), (SSF, 4, 5), (SSF, 1, 1)])
-@pytest.mark.parametrize("kind", ["random", "chain"])
-def test_a_wait_that_is_never_met_ends_the_step(lib, kind, fold, ring, S):
+@pytest.mark.parametrize("kind,place", [("random", 0), ("chain", 0), ("hubs", 0), ("hubs", 4), ("hubs", 6),
+                                        ("chain_hubs", 0), ("chain_hubs", 4)])
+def test_a_wait_that_is_never_met_ends_the_step(lib, kind, place, fold, ring, S):
     net = NETS[kind](4)
-    edges = _edges(net, 0)
+    edges = _edges(net, place)
     for k, edge in enumerate((edges[0], edges[len(edges) // 2], edges[-1])):
         rc, _, _ = run(lib, net, fold, ring, S, seed=k, limit=400, unmet=edge)
         assert rc == 1, (edge, rc)

@@ -283,7 +283,7 @@ __device__ __forceinline__ bool run_sched(const Args& a, const int lane, const i
                 }
                 fold_in<FOLD>(acc1, acc2, qe, f);
             }
-            pass(k, acc1, acc2);
+            if (!stop) pass(k, acc1, acc2);  // (a lane that has given up has no inflow to publish from)
         }
         __builtin_amdgcn_wave_barrier();
         if (many && __any(stop)) {  // (wave-uniform)
