@@ -264,9 +264,10 @@ WFH_HD void kw_terms(const double u, const double dt_dx, const double alpha, dou
     df = u2 * (5.0 * dt_dx * u2 + 3.0 * alpha);
 }
 
-// alpha, dt / dx and the previous discharge such that no term of the updates leaves the normal range
-// (kw_solve bounds C): u starts between 2^-100 and 2^100 and stays below 2^130 then, f and f' lie
-// between 2^-234 and 2^720, and a residual that is divided is above 1e-12.
+// alpha and dt / dx such that, with |C| <= 2^60 (kw_begin) and a start u >= 2^-20 (kw_prepare_dx), no
+// term of the updates leaves the normal range. An update goes up by |C| / f' at most, and f' is at least
+// 3 alpha u^2 >= 2^-69, so u stays below 2^130, f below 2^720 and f' below 2^590. The clamp of the
+// updates keeps u >= 1e-6 > 2^-20, and a residual that is divided is above 1e-12.
 WFH_HD bool kw_range_ok(const double dt_dx, const double alpha) {
     return alpha >= 0x1p-30 && alpha <= 0x1p60 && dt_dx >= 0x1p-30 && dt_dx <= 0x1p60;
 }
@@ -283,7 +284,7 @@ WFH_HD KwPrep kw_prepare_dx(double q_prev, double q_lat, double alpha, double dt
     p.q_lat = q_lat;
     kw_terms(p.u_prev, dt_dx, alpha, p.g0, p.df0);
     p.y0 = wfh_rcp(p.df0);
-    p.fast = range_ok && q_prev >= 0x1p-498 && q_prev <= 0x1p498;
+    p.fast = range_ok && q_prev >= 0x1p-100 && q_prev <= 0x1p498;  // a solve leaves q >= 1e-30 > 2^-100
     return p;
 }
 
@@ -374,10 +375,10 @@ WFH_HD KwRun kw_begin(double q_in, const KwPrep& p, double alpha) {
 // The rest of it, for the lanes with live or any set.
 //
 // A cell whose previous flow is KIN_WAVE_MIN_FLOW starts at u = 1e-6, jumps to about 1e11 and comes
-// down by a fifth per update, about 126 of them. While f(u) + C is above 1024 |C| + 1e-8 the next
-// four updates need no test: an update takes between a tenth and a half off u (f is at least half
-// of f + C, f' at most five and at least three times (f + C) / u), so that f + C falls by less than
-// 7.6-fold in each and every residual stays above |C| + 1e-11, no value repeats and none is
+// down by a fifth per update, about 126 of them. While g = f(u) + C is above 1024 |C| + 1e-8 the next
+// four updates need no test. An update takes f / (u f') of u off, and u f' is between 3 g and 5 g; |C| / g
+// stays below 0.04 over the four, so that each takes between 0.19 and 0.35 of u off and g falls less
+// than 3.6-fold. The residuals in between stay above 20 |C| + 2e-10, no value repeats and none is
 // negative. They run as four bare updates per vote, 95 cycles each instead of 200.
 WFH_HD void kw_end(double q_in, const KwPrep& p, double alpha, KwRun& s) {
     const double dt_dx = p.dt_dx;
@@ -387,7 +388,9 @@ WFH_HD void kw_end(double q_in, const KwPrep& p, double alpha, KwRun& s) {
     int n = 5;  // u is iterate n - 1
     if (s.any) {
         u = p.u_prev > 0.0 ? p.u_prev : wfh_cbrt(C / alpha);
-        if (kw_range_ok(dt_dx, alpha) && wfh_fabs(C) <= 0x1p60 && wfh_fabs(u) >= 0x1p-100 && wfh_fabs(u) <= 0x1p100) {
+        // A start from C: the first update takes at most a fifth of u off (f is dt_dx u^5 there).
+        if (!(p.u_prev > 0.0) && kw_range_ok(dt_dx, alpha) && wfh_fabs(C) <= 0x1p60 && wfh_fabs(u) >= 0x1p-100 &&
+            wfh_fabs(u) <= 0x1p100) {
             n = 1;
             u_p = NaN_;
             kw_terms(u, dt_dx, alpha, g, df);
