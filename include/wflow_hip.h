@@ -378,8 +378,7 @@ int32_t wfh_last_substeps(wfh_handle* h, int32_t* subsurface, int32_t* land, int
  * host memory; WFH_MEM_DEVICE: device memory in land-index order (permuted by a kernel);
  * WFH_MEM_DEVICE_NODE_ORDER: device memory in the library's node order (copied). A device source
  * must be ready when the call is made (synchronise the stream that wrote it); every variant has
- * completed when it returns. When wfh_get reports that a step failed, a device destination may hold
- * the values of that step. */
+ * completed when it returns. When wfh_get reports that a step failed, the destination is unchanged. */
 int32_t wfh_get(wfh_handle* h, int32_t var, double* dst, int64_t count, int32_t memkind);
 int32_t wfh_set(wfh_handle* h, int32_t var, const double* src, int64_t count, int32_t memkind);
 

@@ -1932,6 +1932,12 @@ __global__ void k_scatter(double* out, const double* in, const int* idx, int n) 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) out[idx[i]] = in[i];
 }
+// A read into the caller's device memory, sent behind the step before the host knows how the step
+// ended: a failed step leaves the destination as it is. No index: in the order held.
+__global__ void k_read(double* out, const double* in, const int* idx, size_t n, const int* flags) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && !(flags[0] | flags[1])) out[idx ? idx[i] : i] = in[i];
+}
 
 }  // namespace
 
@@ -4145,14 +4151,28 @@ extern "C" int32_t wfh_set(wfh_handle* h, int32_t var, const double* src, int64_
     return WFH_OK;
 }
 
+// memory of the handle's device, which its kernels can write
+static bool own_memory(wfh_handle* h, const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == h->cfg.device;
+}
+
 static int32_t get_device(wfh_handle* h, int32_t var, double* dst, int64_t count, int32_t memkind) {
     const int64_t n = h->n;
     const bool node = memkind == WFH_MEM_DEVICE_NODE_ORDER;
     VarInfo vi = var_info(h, var);
     const int64_t want = vi.res ? h->nres : vi.river ? h->nriv : n * vi.layers;
-    // The copy goes out behind the step, and one synchronization waits for both; where there is no
-    // copy to send, and before anything is sent on a handle in an error state, the check comes first.
-    if (!vi.p || count != want || count == 0 || h->broken) {
+    const bool direct = vi.res || vi.river || node;  // no permutation
+    // The copy goes out behind the step, as a kernel that copies only if the step has not failed, and
+    // one synchronization waits for both. The check comes first where there is no copy to send, on a
+    // handle in an error state, and where a copy without permutation goes to memory that only the
+    // runtime's copy is known to reach (another device's, the host's).
+    const bool kernel = !direct || own_memory(h, dst);
+    if (!vi.p || count != want || count == 0 || h->broken || !kernel) {
         const int32_t rc = wfh_sync(h);
         if (rc) return rc;
     }
@@ -4170,12 +4190,18 @@ static int32_t get_device(wfh_handle* h, int32_t var, double* dst, int64_t count
     }
     if (count != want) return fail(h, WFH_ERR_ARG, "count mismatch");
     if (count == 0) return WFH_OK;
-    if (vi.res || vi.river || node) {
+    HIPCHK(h, hipSetDevice(h->cfg.device));
+    const int* flags = h->ra.abort_flag;
+    if (!kernel) {
         HIPCHK(h, hipMemcpyAsync(dst, vi.p, (size_t)count * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    } else if (direct) {
+        hipLaunchKernelGGL(k_read, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, h->stream, dst,
+                           (const double*)vi.p, (const int*)nullptr, (size_t)count, flags);
+        HIPCHK(h, hipGetLastError());
     } else {
         for (int k = 0; k < vi.layers; ++k)
-            hipLaunchKernelGGL(k_scatter, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, dst + k * n,
-                               vi.p + k * n, h->d_land_of, (int)n);
+            hipLaunchKernelGGL(k_read, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, dst + k * n,
+                               (const double*)vi.p + k * n, (const int*)h->d_land_of, (size_t)n, flags);
         HIPCHK(h, hipGetLastError());
     }
     return wfh_sync(h);
