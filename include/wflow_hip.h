@@ -362,6 +362,11 @@ int32_t wfh_run(wfh_handle* h, int32_t nsteps, const double* P, const double* E,
  * from the host; node < 0 only sets the limit. */
 int32_t wfh_test_route_stall(wfh_handle* h, int64_t spin_limit, int64_t node);
 
+/* Testing only (no counterpart in the reference): evaluates an elementary function of wfh_math.h on the
+ * device for n pairs of host values. op 0 exp(a), 1 log(a), 2 pow(a, b), 3 cbrt(a), 4 min(a, b), 5 max(a, b),
+ * 6 the in-range quotient a / b (wfh_div_by with wfh_rcp). */
+int32_t wfh_test_math(int32_t device, int32_t op, const double* a, const double* b, double* out, int64_t n);
+
 /* Julian day (1..365; February 29 counts as March 1) that selects the rating-curve column of
  * reservoirs with outflow type 1 in the following steps; 1 after wfh_create. The reference sets
  * it from the step's start time before the river update: julian_day(clock.time - clock.dt).

@@ -3834,6 +3834,43 @@ extern "C" int32_t wfh_test_route_stall(wfh_handle* h, int64_t spin_limit, int64
     return WFH_OK;
 }
 
+// Testing only: the device forms of the elementary functions (wfh_math.h), which tests compare with the
+// host's bit for bit.
+__global__ void k_test_math(int op, const double* a, const double* b, double* out, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double x = a[i], y = b[i];
+    double r = 0.0;
+    switch (op) {
+        case 0: r = wfh_exp(x); break;
+        case 1: r = wfh_log(x); break;
+        case 2: r = wfh_pow(x, y); break;
+        case 3: r = wfh_cbrt(x); break;
+        case 4: r = wfh_min(x, y); break;
+        case 5: r = wfh_max(x, y); break;
+        case 6: r = wfh_div_by(x, y, wfh_rcp(y)); break;
+    }
+    out[i] = r;
+}
+
+extern "C" int32_t wfh_test_math(int32_t device, int32_t op, const double* a, const double* b, double* out, int64_t n) {
+    if (!a || !b || !out || n < 1 || n > (int64_t(1) << 28) || op < 0 || op > 6) return WFH_ERR_ARG;
+    if (hipSetDevice(device) != hipSuccess) return WFH_ERR_HIP;
+    const size_t bytes = (size_t)n * sizeof(double);
+    double* d = nullptr;
+    if (hipMalloc((void**)&d, 3 * bytes) != hipSuccess) return WFH_ERR_HIP;
+    bool ok = hipMemcpy(d, a, bytes, hipMemcpyHostToDevice) == hipSuccess &&
+              hipMemcpy(d + n, b, bytes, hipMemcpyHostToDevice) == hipSuccess;
+    if (ok) {
+        hipLaunchKernelGGL(k_test_math, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, op, (const double*)d,
+                           (const double*)(d + n), d + 2 * n, n);
+        ok = hipGetLastError() == hipSuccess &&
+             hipMemcpy(out, d + 2 * n, bytes, hipMemcpyDeviceToHost) == hipSuccess;
+    }
+    hipFree(d);
+    return ok ? WFH_OK : WFH_ERR_HIP;
+}
+
 // ---- allocation-free step (wfh_step_noalloc) ----
 // The routing scratch of the fixed-sub-step step (ticket counters, abort flag, one outflow slot per
 // cell and sub-step) taken from a fixed device array instead of the handle's allocations. Every

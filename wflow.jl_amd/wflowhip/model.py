@@ -49,6 +49,8 @@ def load_library():
     L.wfh_get_schedule.restype = i32
     L.wfh_test_route_stall.argtypes = [P, i64, i64]
     L.wfh_test_route_stall.restype = i32
+    L.wfh_test_math.argtypes = [i32, i32, P, P, P, i64]
+    L.wfh_test_math.restype = i32
     L.wfh_run.argtypes = [P, i32, P, P, P, P]
     L.wfh_run.restype = i32
     L.wfh_get.argtypes = [P, i32, P, i64, i32]
