@@ -1,0 +1,57 @@
+"""The staged upload of host forcing (wfh_stage.h) on the host: pieces of every size arrive whole and in
+place, a slot is waited for before it is filled again, a failing wait or transfer ends the call with its
+threads, and an allocation or event that could not be made is made by the next call."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = tmp_path_factory.mktemp("stage") / "libstage.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread",
+                    "-I", os.path.join(ROOT, "wflow.jl_amd", "csrc"), "-o", str(out),
+                    os.path.join(HERE, "stage_host.cpp")], check=True)
+    return ctypes.CDLL(str(out))
+
+
+def stage(lib, n, fail_wait=-1, fail_send=-1, wait_us=0):
+    a = np.random.default_rng(n).random(3 * n)
+    out = np.full(3 * n, np.nan)
+    info = np.zeros(4)
+    ok = lib.host_stage(a.ctypes.data_as(ctypes.c_void_p), out.ctypes.data_as(ctypes.c_void_p), ctypes.c_long(n),
+                        fail_wait, fail_send, wait_us, info.ctypes.data_as(ctypes.c_void_p))
+    return ok, a, out, info
+
+
+@pytest.mark.parametrize("n", [1, 7, 2 ** 18 - 1, 2 ** 18, 2 ** 18 + 1, 3 * 2 ** 18 + 5, 1_000_003])
+def test_everything_arrives(lib, n):
+    for wait_us in (0, 50):
+        ok, a, out, info = stage(lib, n, wait_us=wait_us)
+        assert ok == 1 and np.array_equal(a, out) and info[3] == 0
+        assert info[2] == 3 * -(-n // 2 ** 18)
+
+
+@pytest.mark.parametrize("where", ["fail_wait", "fail_send"])
+@pytest.mark.parametrize("piece", [0, 1, 5, 8])
+def test_a_failure_ends_the_call(lib, where, piece):
+    for _ in range(5):
+        ok, a, out, info = stage(lib, 3 * 2 ** 18, **{where: piece})
+        assert ok == 0
+        sent = piece * 2 ** 18
+        assert np.array_equal(a[:sent], out[:sent]) and np.isnan(out[sent:]).all()
+
+
+@pytest.mark.parametrize("fail", [-1, 0, 1, 2, 4])
+def test_what_could_not_be_made_is_made_by_the_next_call(lib, fail):
+    rc, made, count = (ctypes.c_int * 2)(), (ctypes.c_int * 2)(), (ctypes.c_int * 2)()
+    lib.host_ready(fail, rc, made, count)
+    assert list(rc) == [int(fail < 0), 1]
+    assert list(made) == [int(fail < 0), 1]
+    assert list(count) == [1, 4]

@@ -29,13 +29,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "wflow_hip.h"
@@ -43,6 +41,7 @@
 #include "wfh_physics.h"
 #include "wfh_column.h"
 #include "wfh_sched.h"
+#include "wfh_stage.h"
 
 using namespace wfh;
 
@@ -3458,13 +3457,11 @@ static int32_t launch_adaptive(wfh_handle* h) {
 
 // Host forcing of a large grid: the caller's arrays are pageable, and the runtime's own staging copies
 // them with one thread. Here up to HF_THREADS threads copy pieces of HF_SLOT doubles into a ring of
-// pinned slots while the slots before are on their way to the device. All of the arrays has been read
+// pinned slots (wfh_stage.h) while the slots before are on their way to the device. All of the arrays has been read
 // when the call returns; the last transfers may still be under way (hf_copied). Four steps of 1021 x 997
 // cells with host forcing: 14.8 -> 12.9 ms (11.9 of it the kernel); below 2 MiB an array the threads would
 // cost what they save.
 constexpr size_t HF_STAGE_MIN = 2u << 20;  // bytes of one array
-constexpr size_t HF_SLOT = 1u << 18;       // 2 MiB
-constexpr int HF_SLOTS = 4, HF_THREADS = 8;
 
 // memory that the runtime knows nothing of (pinned arrays go straight to the device)
 static bool pageable(const void* p) {
@@ -3477,61 +3474,28 @@ static bool pageable(const void* p) {
 }
 
 static int32_t stage_forcing(wfh_handle* h, const double* const src[3], const size_t n) {
-    if (!h->hf_pin) {
-        if (hipHostMalloc((void**)&h->hf_pin, HF_SLOTS * HF_SLOT * sizeof(double), hipHostMallocDefault) != hipSuccess) {
-            h->hf_pin = nullptr;
-            return fail(h, WFH_ERR_HIP, "hipHostMalloc host-forcing slots");
-        }
-        static_assert(sizeof(h->hf_slot) / sizeof(h->hf_slot[0]) == HF_SLOTS, "an event per slot");
-        for (hipEvent_t& e : h->hf_slot) HIPCHK(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
-    const size_t per = (n + HF_SLOT - 1) / HF_SLOT;  // pieces of an array
-    const int pieces = (int)(3 * per);
-    // A piece is published by its number and copied by all threads, a stripe each.
-    std::atomic<int> go{-1}, done{0};
-    const auto copy = [&](const int i, const int t, const int threads) {
-        const size_t off = (size_t)i % per * HF_SLOT, len = std::min(HF_SLOT, n - off);
-        const size_t a = len * t / threads, b = len * (t + 1) / threads;
-        std::memcpy(h->hf_pin + (size_t)(i % HF_SLOTS) * HF_SLOT + a, src[(size_t)i / per] + off + a,
-                    (b - a) * sizeof(double));
-    };
-    std::thread helpers[HF_THREADS - 1];
-    std::atomic<int> threads{0};  // set once the number of helpers is known
-    int started = 0;
-    const auto work = [&](const int t) {
-        int nt;
-        while ((nt = threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
-        for (int i = 0; i < pieces; ++i) {
-            int g;
-            while ((g = go.load(std::memory_order_acquire)) < i) std::this_thread::yield();
-            if (g >= pieces) return;  // given up
-            copy(i, t, nt);
-            done.fetch_add(1, std::memory_order_release);
-        }
-    };
-    try {
-        for (; started < HF_THREADS - 1; ++started) helpers[started] = std::thread(work, started + 1);
-    } catch (const std::exception&) {  // fewer threads than wanted
-    }
-    const int nt = started + 1;
-    threads.store(nt, std::memory_order_release);
+    static_assert(sizeof(h->hf_slot) / sizeof(h->hf_slot[0]) == HF_SLOTS, "an event per slot");
     hipError_t e = hipSuccess;
-    for (int i = 0; i < pieces && e == hipSuccess; ++i) {
-        const int slot = i % HF_SLOTS;
-        e = hipEventSynchronize(h->hf_slot[slot]);  // (at once if never recorded)
-        if (e != hipSuccess) break;
-        go.store(i, std::memory_order_release);
-        copy(i, 0, nt);
-        while (done.load(std::memory_order_acquire) < (i + 1) * started) std::this_thread::yield();
-        const size_t off = (size_t)i % per * HF_SLOT, len = std::min(HF_SLOT, n - off);
-        e = hipMemcpyAsync(h->hf_tmp + (size_t)i / per * n + off, h->hf_pin + (size_t)slot * HF_SLOT,
-                           len * sizeof(double), hipMemcpyHostToDevice, h->copy_stream);
-        if (e == hipSuccess) e = hipEventRecord(h->hf_slot[slot], h->copy_stream);
-    }
-    if (e != hipSuccess) go.store(pieces, std::memory_order_release);
-    for (int t = 0; t < started; ++t) helpers[t].join();
-    if (e != hipSuccess) return fail(h, WFH_ERR_HIP, std::string("host forcing: ") + hipGetErrorString(e));
-    return WFH_OK;
+    const bool ready = stage_ready(
+        h->hf_pin, h->hf_slot,
+        [&](double*& p) {
+            return (e = hipHostMalloc((void**)&p, HF_SLOTS * HF_SLOT * sizeof(double), hipHostMallocDefault)) == hipSuccess;
+        },
+        [&](hipEvent_t& ev) { return (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) == hipSuccess; });
+    if (ready &&
+        stage_pieces(
+            src, n, h->hf_pin,
+            [&](const int slot) {  // (at once if never recorded)
+                return (e = hipEventSynchronize(h->hf_slot[slot])) == hipSuccess;
+            },
+            [&](const size_t off, const int slot, const size_t len) {
+                e = hipMemcpyAsync(h->hf_tmp + off, h->hf_pin + (size_t)slot * HF_SLOT, len * sizeof(double),
+                                   hipMemcpyHostToDevice, h->copy_stream);
+                if (e == hipSuccess) e = hipEventRecord(h->hf_slot[slot], h->copy_stream);
+                return e == hipSuccess;
+            }))
+        return WFH_OK;
+    return fail(h, WFH_ERR_HIP, std::string("host forcing: ") + hipGetErrorString(e));
 }
 
 extern "C" int32_t wfh_set_forcing(wfh_handle* h, const double* P, const double* E, const double* T,
