@@ -443,9 +443,8 @@ WFH_HD void kw_result(const KwRun& s, double alpha, double& q, double& area) {
     area = s.zero ? 0.0 : alpha * u3;
 }
 
-template <bool DRY = false>
 WFH_HD void kw_solve(double q_in, const KwPrep& p, double alpha, double& q, double& area) {
-    KwRun s = kw_begin<DRY>(q_in, p, alpha);
+    KwRun s = kw_begin<false>(q_in, p, alpha);
     if (WFH_ANY(s.live || s.any)) {
         if (s.live || s.any) kw_end(q_in, p, alpha, s);
     }
