@@ -1,5 +1,6 @@
 // Host run of the staged upload (stage_ready, stage_pieces of wfh_stage.h) for CPU tests: the transfers
 // are copies, and their events, waits and failures are the test's.
+#include <dirent.h>
 #include <sys/resource.h>
 
 #include <chrono>
@@ -10,9 +11,19 @@
 
 using namespace wfh;
 
+static int process_threads() {
+    int n = 0;
+    if (DIR* d = opendir("/proc/self/task")) {
+        while (const dirent* e = readdir(d)) n += e->d_name[0] != '.';
+        closedir(d);
+    }
+    return n;
+}
+
 // Three arrays of n doubles in `in` to `out` [3 n]. Fails the wait or the send of piece fail_wait /
 // fail_send (counted from 0, -1: none); each wait takes wait_us of sleep. info: seconds of CPU time,
-// seconds, pieces sent, a slot sent again before it was waited for (0 / 1). Returns stage_pieces's result.
+// seconds, pieces sent, a slot sent again before it was waited for (0 / 1), threads of the call. Returns
+// stage_pieces's result.
 extern "C" int host_stage(const double* in, double* out, long n, int fail_wait, int fail_send, int wait_us,
                           double* info) {
     const double* const src[3] = {in, in + n, in + 2 * n};
@@ -20,6 +31,8 @@ extern "C" int host_stage(const double* in, double* out, long n, int fail_wait, 
     bool pending[HF_SLOTS] = {};
     int waits = 0, sends = 0;
     bool reused = false;
+    const int before = process_threads();
+    int threads = 0;
     const auto cpu = [] {
         rusage u;
         getrusage(RUSAGE_SELF, &u);
@@ -30,6 +43,7 @@ extern "C" int host_stage(const double* in, double* out, long n, int fail_wait, 
     const bool ok = stage_pieces(
         src, (size_t)n, pin.data(),
         [&](const int slot) {
+            threads = std::max(threads, process_threads() - before + 1);
             if (waits++ == fail_wait) return false;
             if (wait_us > 0) std::this_thread::sleep_for(std::chrono::microseconds(wait_us));
             pending[slot] = false;
@@ -46,6 +60,7 @@ extern "C" int host_stage(const double* in, double* out, long n, int fail_wait, 
     info[1] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     info[2] = sends;
     info[3] = reused;
+    info[4] = threads;
     return ok;
 }
 

@@ -1,6 +1,7 @@
 """The staged upload of host forcing (wfh_stage.h) on the host: pieces of every size arrive whole and in
 place, a slot is waited for before it is filled again, a failing wait or transfer ends the call with its
-threads, and an allocation or event that could not be made is made by the next call."""
+threads, and an allocation or event that could not be made is made by the next call. The call has no
+more threads than CPUs it may use, and they sleep while it waits for transfers."""
 import ctypes
 import os
 import subprocess
@@ -24,7 +25,7 @@ def lib(tmp_path_factory):
 def stage(lib, n, fail_wait=-1, fail_send=-1, wait_us=0):
     a = np.random.default_rng(n).random(3 * n)
     out = np.full(3 * n, np.nan)
-    info = np.zeros(4)
+    info = np.zeros(5)
     ok = lib.host_stage(a.ctypes.data_as(ctypes.c_void_p), out.ctypes.data_as(ctypes.c_void_p), ctypes.c_long(n),
                         fail_wait, fail_send, wait_us, info.ctypes.data_as(ctypes.c_void_p))
     return ok, a, out, info
@@ -55,3 +56,23 @@ def test_what_could_not_be_made_is_made_by_the_next_call(lib, fail):
     assert list(rc) == [int(fail < 0), 1]
     assert list(made) == [int(fail < 0), 1]
     assert list(count) == [1, 4]
+
+
+def test_no_more_threads_than_usable_cpus(lib):
+    cpus = os.sched_getaffinity(0)
+    try:
+        for use in (1, 2, 3):
+            if len(cpus) >= use:
+                os.sched_setaffinity(0, sorted(cpus)[:use])
+                ok, a, out, info = stage(lib, 1_000_003)
+                assert ok == 1 and np.array_equal(a, out)
+                assert info[4] == use
+    finally:
+        os.sched_setaffinity(0, cpus)
+    assert stage(lib, 1_000_003)[3][4] == min(8, len(cpus))
+
+
+def test_threads_sleep_while_the_call_waits(lib):
+    ok, _, _, info = stage(lib, 3 * 2 ** 18, wait_us=30_000)  # nine pieces, a wait of 30 ms before each
+    assert ok == 1 and info[1] > 0.27
+    assert info[0] < 0.5 * info[1], info  # CPU time of all threads; spinning helpers take seven seconds a second
