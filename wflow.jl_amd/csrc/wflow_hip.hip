@@ -3457,11 +3457,15 @@ static int32_t launch_adaptive(wfh_handle* h) {
 
 // Host forcing of a large grid: the caller's arrays are pageable, and the runtime's own staging copies
 // them with one thread. Here up to HF_THREADS threads copy pieces of HF_SLOT doubles into a ring of
-// pinned slots (wfh_stage.h) while the slots before are on their way to the device. All of the arrays has been read
-// when the call returns; the last transfers may still be under way (hf_copied). Four steps of 1021 x 997
-// cells with host forcing: 14.8 -> 12.9 ms (11.9 of it the kernel); below 2 MiB an array the threads would
-// cost what they save.
-constexpr size_t HF_STAGE_MIN = 2u << 20;  // bytes of one array
+// pinned slots (wfh_stage.h) while the slots before are on their way to the device. All of the arrays has
+// been read when the call returns; the last transfers may still be under way (hf_copied). Four steps of
+// 1021 x 997 cells with host forcing: 14.8 -> 12.6 ms (11.9 of it the kernel).
+// The line is where starting the threads costs what they save, for hourly steps that are read each hour,
+// staged / direct, with arrays just written and with arrays last used 600 MB before:
+//    2 MiB an array  1.68 / 1.62  1.63 / 1.61 ms        8 MiB  3.62 / 3.58  3.62 / 3.75 ms
+//    4 MiB           2.20 / 2.14  2.04 / 2.05          12 MiB  4.33 / 4.43  4.21 / 4.48
+//    5.9 MiB         3.00 / 2.96  2.92 / 3.02          32 MiB  8.88 / 9.59  8.39 / 9.21
+constexpr size_t HF_STAGE_MIN = 5u << 20;  // bytes of one array
 
 // memory that the runtime knows nothing of (pinned arrays go straight to the device)
 static bool pageable(const void* p) {
