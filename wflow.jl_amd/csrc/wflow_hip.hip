@@ -1932,10 +1932,17 @@ __global__ void k_scatter(double* out, const double* in, const int* idx, int n) 
     if (i < n) out[idx[i]] = in[i];
 }
 // A read into the caller's device memory, sent behind the step before the host knows how the step
-// ended: a failed step leaves the destination as it is. No index: in the order held.
-__global__ void k_read(double* out, const double* in, const int* idx, size_t n, const int* flags) {
+// ended: a failed step leaves the destination as it is. No index: in the order held. The flags that it
+// looked at go to the host as from k_flags_out, so that a read is one launch and one synchronization.
+__global__ void k_read(double* out, const double* in, const int* idx, size_t n, const int* flags, int* flags_out) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !(flags[0] | flags[1])) out[idx ? idx[i] : i] = in[i];
+    const int f0 = flags[0], f1 = flags[1];
+    if (i < n && !(f0 | f1)) out[idx ? idx[i] : i] = in[i];
+    if (i == 0) {
+        flags_out[0] = f0;
+        flags_out[1] = f1;
+        __threadfence_system();
+    }
 }
 
 }  // namespace
@@ -3942,11 +3949,8 @@ extern "C" int32_t wfh_set_julian_day(wfh_handle* h, int32_t julian_day) {
     return WFH_OK;
 }
 
-extern "C" int32_t wfh_sync(wfh_handle* h) {
-    if (!h) return WFH_ERR_ARG;
-    HIPCHK(h, hipSetDevice(h->cfg.device));
-    hipLaunchKernelGGL(k_flags_out, dim3(1), dim3(1), 0, h->stream, (const int*)h->ra.abort_flag, h->flags_host);
-    HIPCHK(h, hipGetLastError());
+// Waits for the handle's stream, where a launch has written the error flags to flags_host, and checks them.
+static int32_t wait_checked(wfh_handle* h) {
     HIPCHK(h, hipStreamSynchronize(h->stream));
     const int* flag = h->flags_host;
     if (flag[1]) {
@@ -3960,6 +3964,14 @@ extern "C" int32_t wfh_sync(wfh_handle* h) {
         return fail(h, WFH_ERR_DEVICE, "routing kernel aborted: a dependency wait exceeded its spin limit");
     }
     return WFH_OK;
+}
+
+extern "C" int32_t wfh_sync(wfh_handle* h) {
+    if (!h) return WFH_ERR_ARG;
+    HIPCHK(h, hipSetDevice(h->cfg.device));
+    hipLaunchKernelGGL(k_flags_out, dim3(1), dim3(1), 0, h->stream, (const int*)h->ra.abort_flag, h->flags_host);
+    HIPCHK(h, hipGetLastError());
+    return wait_checked(h);
 }
 
 namespace {
@@ -4196,20 +4208,17 @@ static int32_t get_device(wfh_handle* h, int32_t var, double* dst, int64_t count
     if (count != want) return fail(h, WFH_ERR_ARG, "count mismatch");
     if (count == 0) return WFH_OK;
     HIPCHK(h, hipSetDevice(h->cfg.device));
-    const int* flags = h->ra.abort_flag;
     if (!kernel) {
         HIPCHK(h, hipMemcpyAsync(dst, vi.p, (size_t)count * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
-    } else if (direct) {
-        hipLaunchKernelGGL(k_read, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, h->stream, dst,
-                           (const double*)vi.p, (const int*)nullptr, (size_t)count, flags);
-        HIPCHK(h, hipGetLastError());
-    } else {
-        for (int k = 0; k < vi.layers; ++k)
-            hipLaunchKernelGGL(k_read, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, dst + k * n,
-                               (const double*)vi.p + k * n, (const int*)h->d_land_of, (size_t)n, flags);
-        HIPCHK(h, hipGetLastError());
+        return wfh_sync(h);
     }
-    return wfh_sync(h);
+    const int64_t len = direct ? count : n;  // values of a launch
+    for (int64_t k = 0; k < count; k += len)
+        hipLaunchKernelGGL(k_read, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, h->stream, dst + k,
+                           (const double*)vi.p + k, (const int*)(direct ? nullptr : h->d_land_of), (size_t)len,
+                           (const int*)h->ra.abort_flag, h->flags_host);
+    HIPCHK(h, hipGetLastError());
+    return wait_checked(h);
 }
 
 static int32_t set_device(wfh_handle* h, int32_t var, const double* src, int64_t count, int32_t memkind) {
